@@ -121,13 +121,15 @@ struct psba_ctx {
   double* ref_part = nullptr;  // 2 cnp per camera chunk
   long ref_part_cap = 0;
   int refine_steps = 0;        // sweeps per trial (psba_opts.refine_steps)
-  // fused factor + solve (k_chol_solve): factor, right-hand side copy, y = L^-1 b,
-  // bar = [grid-barrier counter (only grows), x flag, T row flags, epoch
-  // (the counter's value before the next launch)]
-  double *Lf = nullptr, *bw = nullptr, *yv = nullptr;
-  unsigned long long* bar = nullptr;
+  // fused factor + solve: the factor and scratch of the solve; FP64 (k_chol_solve):
+  // the diagonal tiles' inverses (their unwritten upper parts stay zero) and the
+  // flags between workgroups (they only grow); mixed (k_chol_phases): right-hand
+  // side copy and bar = [grid-barrier counter (only grows), x flag, T row flags,
+  // epoch (the counter's value before the next launch)]
+  double *Lf = nullptr, *yv = nullptr, *Minv = nullptr, *bw = nullptr;
+  unsigned long long *sync = nullptr, *bar = nullptr;
   int* chol_fail = nullptr;
-  int chol_grid = 0, chol_resident = 0;
+  int chol_grid = 0;
   const double* L_cur = nullptr;  // where the last factor lives (Lf, or S after the modified Cholesky)
   double* Saux = nullptr;      // copy of S for the dogleg's recovery path (allocated on first use)
   double* snap = nullptr;      // parameter snapshot (psba_snapshot_params)
@@ -188,6 +190,11 @@ int launch_schur(psba_ctx* c, double mu);                 // S (lower), ea
 int build_point_order(psba_ctx* c);                        // pt_order (index builds)
 int build_schur_slots(psba_ctx* c);                        // slot_items, cchunk_rec (index builds)
 int launch_ea_rhs(psba_ctx* c, const double* ga, const double* z, double* out);  // ga - sum W z
+
+// ---- launchers (k_chol.hip) ----
+int launch_chol(psba_ctx* c);  // launch_factor_solve of an FP64 context
+long chol_sync_words(int T);   // lengths of ctx->sync and ctx->Minv for T tiles a side
+long chol_inv_len(int T);
 
 // ---- launchers (k_dense.hip) ----
 int launch_factor_solve(psba_ctx* c);                     // S -> Lf, SC_FACTOR_OK; dp[0..n) = S^-1 ea

@@ -228,9 +228,15 @@ int psba_create(const psba_desc* d, psba_ctx** out) {
   chk(dalloc(&c->vecD, (size_t)c->ntot));
   chk(dalloc(&c->mc_work, 3 * (size_t)c->n_pad));
   chk(dalloc(&c->Lf, (size_t)c->n_pad * c->n_pad));
-  chk(dalloc(&c->bw, (size_t)c->n_pad));
   chk(dalloc(&c->yv, (size_t)c->n_pad));
-  chk(dalloc(&c->bar, (size_t)3 + (size_t)(c->n_pad / kNB)));  // barrier counter, back-substitution flags, epoch
+  const int T = (int)(c->n_pad / kNB);
+  if (c->mixed()) {
+    chk(dalloc(&c->bw, (size_t)c->n_pad));
+    chk(dalloc(&c->bar, (size_t)3 + T));
+  } else {
+    chk(dalloc(&c->sync, (size_t)chol_sync_words(T)));
+    chk(dalloc(&c->Minv, (size_t)chol_inv_len(T)));
+  }
   chk(dalloc(&c->chol_fail, (size_t)1));
   c->red_part_cap = 8 * (long)std::max(ceil_div(c->no, 256), ceil_div(c->ntot, 256)) + 64;
   chk(dalloc(&c->red_part, (size_t)c->red_part_cap));
@@ -248,7 +254,12 @@ int psba_create(const psba_desc* d, psba_ctx** out) {
     z(hipMemsetAsync(c->dp, 0, sizeof(double) * (size_t)c->ntot, c->stream));
     z(hipMemsetAsync(c->d_scal, 0, sizeof(double) * SC_COUNT, c->stream));
     z(hipMemsetAsync(c->chol_fail, 0, sizeof(int), c->stream));
-    z(hipMemsetAsync(c->bar, 0, sizeof(unsigned long long) * (3 + (size_t)(c->n_pad / kNB)), c->stream));
+    if (c->mixed()) {
+      z(hipMemsetAsync(c->bar, 0, sizeof(unsigned long long) * ((size_t)3 + T), c->stream));
+    } else {
+      z(hipMemsetAsync(c->sync, 0, sizeof(unsigned long long) * (size_t)chol_sync_words(T), c->stream));
+      z(hipMemsetAsync(c->Minv, 0, sizeof(double) * (size_t)chol_inv_len(T), c->stream));
+    }
     z(hipMemsetAsync(c->Lf, 0, sizeof(double) * (size_t)c->n_pad * c->n_pad, c->stream));
     if (c->n_pad > c->n)
       hipLaunchKernelGGL(k_pad_identity, dim3(1), dim3(64), 0, c->stream, c->S, c->n_pad, c->n, c->n_pad);
@@ -272,7 +283,7 @@ int psba_destroy(psba_ctx* c) {
   double* bufs[] = {c->K, c->q0, c->meas, c->cams, c->pts, c->e, c->JA, c->JB, c->W, c->U, c->V, c->g,
                     c->uvdiag, c->Vinv, c->z, c->S, c->ea, c->xsol, c->dp, c->eb, c->vecA, c->vecB,
                     c->vecC, c->vecD, c->mc_work, c->red_part, c->d_scal, c->Saux, c->snap,
-                    c->Lf, c->bw, c->yv};
+                    c->Lf, c->Minv, c->bw, c->yv};
   for (double* p : bufs)
     if (p) (void)hipFree(p);
   dfree(c->fix);
@@ -282,6 +293,7 @@ int psba_destroy(psba_ctx* c) {
   dfree(c->W32);
   dfree(c->ref_obs);
   dfree(c->ref_part);
+  dfree(c->sync);
   dfree(c->bar);
   dfree(c->chol_fail);
   if (c->lm) (void)hipFree(c->lm);

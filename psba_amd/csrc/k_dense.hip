@@ -1,7 +1,8 @@
 // Dense FP64 linear algebra on the reduced camera matrix S (n_pad x n_pad,
 // row-major, lower triangle; rows/cols >= n are the identity):
 //   - Cholesky S = L L^T and the solve S dpa = e_a fused in one cooperative
-//     launch over 64x64 tiles (k_chol_solve below); replaces the reference's
+//     launch over 64x64 tiles: k_chol_phases below for mixed-precision contexts,
+//     k_chol_solve (k_chol.hip) for the others; they replace the reference's
 //     explicit inverse (PSBA/CL_files/SPD_inv.cl, kern_cholesky/_s2 +
 //     kern_trigMat_inv/_mul + kern_fill_rest) and matVec_mul.cl;
 //   - the dogleg's modified Cholesky and lambda = |sum E| / n
@@ -223,7 +224,14 @@ int launch_modchol(psba_ctx* c, double* A) {
 }
 
 // ---------------------------------------------------------------------------
-// Fused Cholesky factor and solve of S dpa = e_a in ONE launch.
+// Fused Cholesky factor and solve of S dpa = e_a in ONE launch, for mixed
+// precision.  (FP64 contexts take k_chol_solve, which is about twice as fast.
+// In a mixed-precision solve's last trials the system is singular to FP32
+// accuracy along its free scale, so that a difference of 1e-16 in a step decides
+// single FP32 roundings of the next assembly and grows to 1e-5 .. 1e-4 of the
+// points by the end -- measured on five of six 88-camera scenes, as often
+// towards the minimum as away from it.  These solves keep the arithmetic, and
+// with it the results, that they have always had.)
 //
 // S is viewed as T x T tiles of 64 (T = n_pad / 64).  Phase k (k = 0..T-2)
 // applies panel k to the trailing matrix: for every tile (i, j) with
@@ -965,7 +973,7 @@ __device__ __forceinline__ double tile_matvec(CholSmem& sm, const double* Lt, in
   return t;
 }
 
-// One forward step of k_chol_solve's forward workgroup in phase k >= 1:
+// One forward step of k_chol_phases' forward workgroup in phase k >= 1:
 // b_i -= L_{i,k-1} y_{k-1} for i = k..T-1 (y_{k-1} in sm.w; from yv at k = 1,
 // where workgroup 0 formed it), then y_k = L_kk^-1 b_k into yv and sm.w.
 // Thread (lane, w) takes row `lane`, columns 16w..16w+15 of each tile; four
@@ -1019,7 +1027,7 @@ __device__ void forward_step(CholSmem& sm, const double* __restrict__ Lf, int ld
   __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void k_chol_solve(double* __restrict__ A, int ld, int T, double* __restrict__ Lf,
+__global__ __launch_bounds__(256) void k_chol_phases(double* __restrict__ A, int ld, int T, double* __restrict__ Lf,
                                                     const double* __restrict__ ea, double* __restrict__ bw,
                                                     double* __restrict__ yv, double* __restrict__ xs,
                                                     double* __restrict__ dp, int n, double* __restrict__ ok,
@@ -1393,24 +1401,25 @@ int launch_tri_solve(psba_ctx* c, const double* b, double* out) {
 }
 
 int launch_factor_solve(psba_ctx* c) {
+  if (!c->mixed()) return launch_chol(c);
   const int T = c->n_pad / NB;
   if (c->chol_grid <= 0) {
     int per_cu = 0, ncu = 0;
-    PSBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_chol_solve, 256, 0));
+    PSBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_chol_phases, 256, 0));
     PSBA_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
     // at most one workgroup per CU (the LDS use allows no more), so that every
     // workgroup of a launch is resident at once on the stream's device
-    c->chol_resident = std::min(per_cu, 1) * ncu;
-    if (c->chol_resident < 1) return PSBA_ERR_UNSUPPORTED;
+    const int resident = std::min(per_cu, 1) * ncu;
+    if (resident < 1) return PSBA_ERR_UNSUPPORTED;
     // one workgroup per task of the first phase, and one more for the forward
     // substitution when there are at least three tiles
-    c->chol_grid = std::max(1, std::min(c->chol_resident, (T - 1) * T / 2 + (T >= 3 ? 1 : 0)));
+    c->chol_grid = std::max(1, std::min(resident, (T - 1) * T / 2 + (T >= 3 ? 1 : 0)));
   }
   int G = c->chol_grid;
   double* ok = c->d_scal + SC_FACTOR_OK;
   int ld = c->n_pad, n = c->n;
   probe_begin(c, PSBA_PROBE_FACTOR);
-  hipLaunchKernelGGL(k_chol_solve, dim3(G), dim3(256), 0, c->stream, c->S, ld, T, c->Lf, c->ea, c->bw, c->yv,
+  hipLaunchKernelGGL(k_chol_phases, dim3(G), dim3(256), 0, c->stream, c->S, ld, T, c->Lf, c->ea, c->bw, c->yv,
                      c->xsol, c->dp, n, ok, c->bar, c->chol_fail, gate_of(c, kGateActive));
   probe_end(c, PSBA_PROBE_FACTOR);
   c->L_cur = c->Lf;
@@ -1422,7 +1431,7 @@ int launch_factor_solve(psba_ctx* c) {
 
 // ---------------------------------------------------------------------------
 // batched problems: one workgroup factors and solves one problem's reduced
-// system with the same tile tasks as k_chol_solve, run in sequence (the
+// system with the same tile tasks as k_chol_phases, run in sequence (the
 // diagonal task of each phase last, so its factor stays in LDS for the next
 // phase).  Arithmetic per tile is the same as in the single-problem kernel.
 // ---------------------------------------------------------------------------
@@ -1510,7 +1519,7 @@ __global__ __launch_bounds__(256) void k_b_chol_solve(double* __restrict__ S, do
     }
   }
 
-  // back substitution, right-looking as in k_chol_solve: step k applies
+  // back substitution, right-looking as in k_chol_phases: step k applies
   // x_{k+1} (in sm.w) to r_k, solves x_k, then applies x_{k+1} to r_i, i < k
   for (int k = T - 1; k >= 0; --k) {
     load_lower(sm.P, tile(L, k, k), ld);

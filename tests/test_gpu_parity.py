@@ -261,6 +261,30 @@ def test_dense_factor_solve_matches_lapack(P, gpu, n_cams):
         assert rel(np.tril(L), np.linalg.cholesky(S)) < 1e-11
 
 
+# one tile (padded, full), two and three tiles at their edges, the last size with a
+# workgroup per tile and the first with several tiles each (256 compute units), more of those
+@pytest.mark.parametrize("cnp,n_cams", [(16, 4), (16, 8), (11, 12), (16, 12), (16, 88), (16, 89), (9, 300)])
+def test_dense_factor_at_tile_edges(P, gpu, cnp, n_cams):
+    rng = np.random.default_rng(n_cams)
+    n = cnp * n_cams
+    S = spd(n, rng)
+    b = rng.standard_normal(n)
+    junk = np.tril(S) + np.triu(np.full((n, n), np.nan), 1)
+    bad = junk.copy()
+    bad[n // 2, n // 2] = -1.0
+    with P.Context(cnp, n_cams, 4, 8) as c:
+        runs = []
+        for A, good in [(junk, True), (bad, False), (junk, True)]:
+            c.load_S(A, b)
+            ok, x = c.factor_only()
+            assert ok == good
+            runs.append((x.copy(), np.tril(c.buffer("L").reshape(n, n))))
+    assert np.array_equal(runs[0][0], runs[2][0]) and np.array_equal(runs[0][1], runs[2][1])
+    x, L = runs[0]
+    assert rel(x, np.linalg.solve(S, b)) < 1e-9
+    assert rel(L, np.linalg.cholesky(S)) < 1e-11
+
+
 @pytest.mark.parametrize("n_cams", [7, 40])
 def test_dense_factor_reads_the_lower_triangle_only(P, gpu, n_cams):
     """The Schur assembly writes only the lower block positions of S, so the
