@@ -294,6 +294,15 @@ int launch_round(psba_batch* b) {
   return PSBA_OK;
 }
 
+// what was read ahead is no longer what the device holds
+void drop_read_ahead(psba_batch* b) {
+  std::lock_guard<std::mutex> lock(b->ahead_mtx);
+  b->ahead_lo = b->ahead_hi = 0;
+  b->last_slot = -1;
+}
+
+constexpr size_t kReadAhead = (size_t)4 << 20;  // bytes of results fetched together
+
 // wait for the rounds queued behind the last check and read the solve's time
 int settle(psba_batch* b) {
   if (!b->stop_pending) return PSBA_OK;
@@ -743,6 +752,7 @@ int psba_batch_commit(psba_batch* b) {
   PSBA_HIP_TRY(hipMemsetAsync(b->dp, 0, sizeof(double) * (size_t)(z.N + 3 * z.NP), b->stream));
   b->committed = true;
   b->finished = false;
+  drop_read_ahead(b);
   return PSBA_OK;
 }
 
@@ -758,6 +768,7 @@ int psba_batch_launch(psba_batch* b, const psba_opts* o) {
   b->max_rounds = b->max_iter * 31 + 2;
   PSBA_TRY(capture_round(b));
   b->stop_pending = false;  // an unread time of the previous solve is dropped
+  drop_read_ahead(b);
   PSBA_HIP_TRY(hipEventRecord(b->ev_start, b->stream));
   PSBA_HIP_TRY(hipMemcpyAsync(b->cams, b->cams0, sizeof(double) * (size_t)b->N, hipMemcpyDeviceToDevice, b->stream));
   PSBA_HIP_TRY(
@@ -807,13 +818,39 @@ int psba_batch_result(psba_batch* b, int slot, int* code, int* itno, double* ini
   if (itno) *itno = st.itno;
   if (init_err) *init_err = st.init_err;
   if (final_err) *final_err = st.cost;
-  const int C = b->cnp;
-  if (cams)
-    PSBA_HIP_TRY(hipMemcpy(cams, b->cams + (size_t)C * b->h_cam_off[slot],
-                           sizeof(double) * C * (b->h_cam_off[slot + 1] - b->h_cam_off[slot]), hipMemcpyDeviceToHost));
-  if (pts)
-    PSBA_HIP_TRY(hipMemcpy(pts, b->pts + 3 * (size_t)b->h_pt_off[slot],
-                           sizeof(double) * 3 * (b->h_pt_off[slot + 1] - b->h_pt_off[slot]), hipMemcpyDeviceToHost));
+  if (!cams && !pts) return PSBA_OK;
+  const size_t C = (size_t)b->cnp, N = (size_t)b->N;
+  const size_t c0 = C * b->h_cam_off[slot], c1 = C * b->h_cam_off[slot + 1];
+  const size_t p0 = 3 * (size_t)b->h_pt_off[slot], p1 = 3 * (size_t)b->h_pt_off[slot + 1];
+  std::lock_guard<std::mutex> lock(b->ahead_mtx);
+  double* const image = (double*)b->staging;
+  if (slot < b->ahead_lo || slot >= b->ahead_hi) {
+    if (slot != b->last_slot + 1 || slot == 0) {
+      b->last_slot = slot;
+      if (cams) PSBA_HIP_TRY(hipMemcpy(cams, b->cams + c0, sizeof(double) * (c1 - c0), hipMemcpyDeviceToHost));
+      if (pts) PSBA_HIP_TRY(hipMemcpy(pts, b->pts + p0, sizeof(double) * (p1 - p0), hipMemcpyDeviceToHost));
+      return PSBA_OK;
+    }
+    // one slot after another: this one and the next, up to kReadAhead bytes.  Two
+    // copies a slot into pageable memory took 40 us a slot (512 windows: 20 of 48 ms).
+    int hi = slot + 1;
+    auto bytes = [&](int h) {
+      return sizeof(double) * (C * (size_t)(b->h_cam_off[h] - b->h_cam_off[slot]) +
+                               3 * (size_t)(b->h_pt_off[h] - b->h_pt_off[slot]));
+    };
+    while (hi < b->P && bytes(hi + 1) <= kReadAhead) ++hi;
+    b->ahead_lo = b->ahead_hi = 0;
+    const size_t c2 = C * b->h_cam_off[hi], p2 = 3 * (size_t)b->h_pt_off[hi];
+    PSBA_HIP_TRY(hipMemcpyAsync(image + c0, b->cams + c0, sizeof(double) * (c2 - c0), hipMemcpyDeviceToHost, b->stream));
+    PSBA_HIP_TRY(
+        hipMemcpyAsync(image + N + p0, b->pts + p0, sizeof(double) * (p2 - p0), hipMemcpyDeviceToHost, b->stream));
+    PSBA_HIP_TRY(hipStreamSynchronize(b->stream));
+    b->ahead_lo = slot;
+    b->ahead_hi = hi;
+  }
+  b->last_slot = slot;
+  if (cams) std::copy(image + c0, image + c1, cams);
+  if (pts) std::copy(image + N + p0, image + N + p1, pts);
   return PSBA_OK;
 }
 
@@ -832,6 +869,7 @@ int psba_batch_autotune(psba_batch* b, int* obs_block, int* pt_block) {
   if (b->running) return bfail(PSBA_ERR_STATE, "a solve is in flight");
   PSBA_HIP_TRY(hipSetDevice(b->device));
   PSBA_TRY(settle(b));
+  drop_read_ahead(b);
   // state as at the start of a solve: every problem needs its Jacobian
   b->max_iter = 100;
   PSBA_HIP_TRY(hipMemcpyAsync(b->cams, b->cams0, sizeof(double) * (size_t)b->N, hipMemcpyDeviceToDevice, b->stream));

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -62,6 +63,11 @@ struct psba_batch {
   char* staging = nullptr;
   size_t staging_bytes = 0;
   hipEvent_t ev_staged = nullptr;
+  // results read ahead (psba_batch_result): the parameters of slots [ahead_lo,
+  // ahead_hi) of the finished solve, in the staging image at the places that cams
+  // and pts have from its start; last_slot: the one asked for last
+  std::mutex ahead_mtx;
+  int ahead_lo = 0, ahead_hi = 0, last_slot = -1;
 
   // problem data
   double *K = nullptr, *q0 = nullptr, *meas = nullptr, *cams = nullptr, *pts = nullptr;

@@ -261,3 +261,28 @@ def test_eager_rounds_equal_graph_rounds(P, gpu, monkeypatch):
     eager = solve_batch(P, scenes)
     for a, b in zip(graph, eager):
         same(a, b)
+
+
+@pytest.mark.parametrize("n_pts", [(3,), (40, 7, 300), (40000, 30000, 60000, 200, 50000, 180000, 40000)])
+def test_results_in_order_equal_results_out_of_order(P, gpu, n_pts):
+    """Slots read one after another come in groups of a few MB (one larger slot
+    alone); slots read in descending order one by one.  A later solve's results
+    replace what was read ahead."""
+    scenes = [window(P, k, n_cams=5, n_pts=n) for k, n in enumerate(n_pts)]
+    b = P.Batch(6)
+    for sc in scenes:
+        b.add_scene(sc)
+    b.commit()
+    first = None
+    for iters in (2, 4):
+        b.solve(max_iter=iters)
+        up = [b.result(s) for s in range(len(scenes))]
+        down = [b.result(s) for s in reversed(range(len(scenes)))][::-1]
+        again = [b.result(s) for s in range(len(scenes))]
+        for u, d, a in zip(up, down, again):
+            same(u, d)
+            same(u, a)
+        if first:
+            assert any(not np.array_equal(u["pts"], f["pts"]) for u, f in zip(up, first))
+        first = up
+    b.close()
