@@ -365,6 +365,21 @@ __device__ __forceinline__ void solve_rows(dvec4 (&xt)[4], const double (&av)[16
   }
 }
 
+// its 16-column block MB alone
+template <int MB>
+__device__ __forceinline__ void solve_block(dvec4& xt, const double (&av)[16], const lds_dbl* frag) {
+  const int lane = threadIdx.x & 63;
+  xt = dvec4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int kb = 0; kb <= MB; ++kb)
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const dvec2 f = ((const lds_dvec2*)frag)[inv_block(MB, kb) * 128 + s2 * 64 + lane];
+      xt = mfma(f[0], av[4 * kb + 2 * s2], xt);
+      xt = mfma(f[1], av[4 * kb + 2 * s2 + 1], xt);
+    }
+}
+
 // A tile from global memory straight to LDS as operand fragments (no registers,
 // in flight until vmcnt says otherwise): pairs at ((rb * 4 + kb) * 2 + s / 2) * 64 + l
 // for rows 16 rb + l % 16.  Chunks c0, c0 + step, .. of the 32, one wave each.

@@ -23,13 +23,13 @@
 // (factor 7.0, the rest of M_k 0.8, L_{k+1,k} 1.5, its product 2.2), then 1.8 us
 // a tile back.  Workgroups that met at a barrier after each phase, with solves
 // by substitution, took 14.5 us a phase and more: 117 us at n = 300, 230 at 594,
-// 323 at 828, 1916 at 2700; this kernel takes 69, 138, 182 and 965.
+// 323 at 828, 1916 at 2700; this kernel takes 69, 138, 183 and 700.
 //
 // With more tiles than workgroups (T > 22 on 256 compute units) an owner has
-// several tiles and keeps them in memory: then the solves are not repeated per
-// tile, but go through memory once; with one tile each,
-// repeating them saves a hop between workgroups (14.3 us a tile at T = 22, which
-// the first form would take 15.3 for).
+// several tiles: then the solves are not repeated per tile, but go through memory
+// once, and kForward workgroups share the forward substitution.  With one tile
+// each, repeating the solves saves a hop between workgroups: 14.1 us a tile at
+// T = 22, 15.1 at T = 24.
 //
 // Every wait is for one flag (a word that only grows: done is the launch's epoch
 // plus one, so nothing is reset between launches), set by its producer behind a
@@ -49,16 +49,18 @@ namespace {
 
 typedef unsigned long long ull;
 
-// Words of the sync array: epoch, x flag, M flags (T), r flags (T), then A and L
-// flags of the lower tiles, row by row.
+// Words of the sync array: epoch, x and y flags, M flags (T), r and s flags (T each),
+// then A and L flags of the lower tiles, row by row.
 struct Sync {
   ull* w;
   int T;
   __device__ __forceinline__ ull* epoch() const { return w; }
   __device__ __forceinline__ ull* x() const { return w + 1; }
-  __device__ __forceinline__ ull* m(int k) const { return w + 2 + k; }
-  __device__ __forceinline__ ull* r(int k) const { return w + 2 + T + k; }
-  __device__ __forceinline__ ull* a(int i, int j) const { return w + 2 + 2 * T + i * (i + 1) / 2 + j; }
+  __device__ __forceinline__ ull* y() const { return w + 2; }
+  __device__ __forceinline__ ull* m(int k) const { return w + 3 + k; }
+  __device__ __forceinline__ ull* r(int k) const { return w + 3 + T + k; }
+  __device__ __forceinline__ ull* s(int k) const { return w + 3 + 2 * T + k; }
+  __device__ __forceinline__ ull* a(int i, int j) const { return w + 3 + 3 * T + i * (i + 1) / 2 + j; }
   __device__ __forceinline__ ull* l(int i, int j) const { return a(i, j) + T * (T + 1) / 2; }
 };
 
@@ -89,12 +91,13 @@ __device__ __forceinline__ void wait_flags(ull v, int* fail, ull* f0, ull* f1 = 
   __syncthreads();
 }
 
-// After the workgroup's stores: make them visible and set the flag.
-__device__ __forceinline__ void publish(ull* f, ull v) {
+// After the workgroup's stores: make them visible and set the flags (null: none).
+__device__ __forceinline__ void publish(ull* f0, ull v, ull* f1 = nullptr) {
   __syncthreads();  // every wave's stores have been accepted
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (f0) __hip_atomic_store(f0, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (f1) __hip_atomic_store(f1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -140,19 +143,24 @@ struct SolveLds {
 static_assert(2 * NB * TS >= kMaxSolveN, "the right-hand side must fit");
 
 constexpr int kInvLen = kInvFrag + NB * NB;  // what is stored of M_k: fragments, then row-major
-constexpr int kNear = 3;  // terms x_{k+1} .. x_{k+3} of row k are workgroup 1's
+constexpr int kNear = 3;  // the terms of row k's three neighbours are workgroup 1's
+// With more tiles than workgroups, so many workgroups take the far terms of the
+// forward substitution: one workgroup reads tiles at about 60 GB/s, which left it
+// behind the factorisation by 100 of 965 us at T = 43
+constexpr int kForward = 8;
+constexpr int kHeld = 4;  // and so many tiles an owner keeps in registers
 
 // the tile's accumulators: wave w has rows 16 w .. + 15, acc[c] columns 16 c .. + 15
-__device__ __forceinline__ void acc_load(dvec4 (&acc)[4], const double* A, int ld) {
-  const int lane = threadIdx.x & 63, w = wave_id(), li = lane & 15, lk = lane >> 4;
+__device__ __forceinline__ void acc_load(dvec4 (&acc)[4], const double* A, int ld, int w) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll
   for (int c = 0; c < 4; ++c)
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[c][r] = A[(size_t)(16 * w + 4 * r + lk) * ld + 16 * c + li];
 }
 
-__device__ __forceinline__ void acc_store(const dvec4 (&acc)[4], double* A, int ld) {
-  const int lane = threadIdx.x & 63, w = wave_id(), li = lane & 15, lk = lane >> 4;
+__device__ __forceinline__ void acc_store(const dvec4 (&acc)[4], double* A, int ld, int w) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll
   for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -177,9 +185,10 @@ __device__ __forceinline__ void acc_update(dvec4 (&acc)[4], const dvec4 (&x)[4],
     }
 }
 
-// fragments of M_k from global memory into LDS
+// fragments of M_k from global memory into LDS, by the workgroup's first 256 threads
 __device__ __forceinline__ void load_inv(lds_dbl* F, const double* M) {
   dvec2 t[5];
+  if (threadIdx.x >= 256) return;
 #pragma unroll
   for (int q = 0; q < 5; ++q) t[q] = ((const dvec2*)M)[threadIdx.x + 256 * q];
 #pragma unroll
@@ -187,8 +196,8 @@ __device__ __forceinline__ void load_inv(lds_dbl* F, const double* M) {
 }
 
 // L_ij of the wave's sixteen rows, from its result fragments
-__device__ __forceinline__ void store_rows(const dvec4 (&xt)[4], double* L, int ld) {
-  const int lane = threadIdx.x & 63, w = wave_id(), li = lane & 15, lk = lane >> 4;
+__device__ __forceinline__ void store_rows(const dvec4 (&xt)[4], double* L, int ld, int w) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -455,6 +464,42 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
     return;
   }
 
+  const int ntiles = T * (T - 1) / 2 + max(0, T - 2);
+  const bool many = ntiles > G - 2;  // more tiles than workgroups
+  // eight waves: row i's share of b (rows i0, i0 + step, .. below i1; row i
+  // lies at place i / step) -= L_ik y, with the next two tiles'
+  // loads in flight
+  auto forward = [&](lds_dbl* b, lds_dbl* y, int k, int i0, int step, int i1) {
+    for (int j0 = i0; j0 < i1; j0 += 64 * step) {
+      const int j1 = min(j0 + 64 * step, i1);
+      if (w == 0) {
+        if (j0 + lane * step < j1) poll(sy.l(j0 + lane * step, k), done, fail);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      __syncthreads();
+      TileRegs<8> t[2][2];
+      auto load = [&](int s, int i) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (i + u * step < j1) t[s][u].load(tile(Lf, i + u * step, k), ld);
+      };
+      auto take = [&](int s, int i) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (i + u * step < j1) t[s][u].rows(y, (lds_dbl*)sm.part[s][u]);
+        __syncthreads();
+        if (w < 2 && i + w * step < j1) b[(i + w * step) / step * NB + lane] -= sm.part[s][w][lane];
+      };
+      load(0, j0);
+      for (int i = j0; i < j1; i += 4 * step) {
+        load(1, i + 2 * step);
+        take(0, i);
+        load(0, i + 4 * step);
+        take(1, i + 2 * step);
+      }
+    }
+  };
+
   if (blockIdx.x == 1) {
     // ---- the triangular solves.  b holds b_i, then y_i, then x_i.
     lds_dbl* const b = (lds_dbl*)&sm.Y[0][0];
@@ -473,34 +518,20 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
       }
       __syncthreads();
       if (w == 0) b[k * NB + lane] = y[lane];
-      // b_i -= L_ik y_k, the next two tiles' loads in flight
-      for (int i0 = k + 1; i0 < T; i0 += 64) {
-        const int i1 = min(i0 + 64, T);
+      if (many) {
         if (w == 0) {
-          if (i0 + lane < i1) poll(sy.l(i0 + lane, k), done, fail);
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+          xs[(size_t)k * NB + lane] = y[lane];
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+          if (lane == 0) __hip_atomic_store(sy.y(), epoch + (ull)(k + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();
-        TileRegs<8> t[2][2];
-        auto load = [&](int s, int i) {
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-            if (i + u < i1) t[s][u].load(tile(Lf, i + u, k), ld);
-        };
-        auto take = [&](int s, int i) {
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-            if (i + u < i1) t[s][u].rows(y, (lds_dbl*)sm.part[s][u]);
-          __syncthreads();
-          if (w < 2 && i + w < i1) b[(i + w) * NB + lane] -= sm.part[s][w][lane];
-        };
-        load(0, i0);
-        for (int i = i0; i < i1; i += 4) {
-          load(1, i + 2);
-          take(0, i);
-          load(0, i + 4);
-          take(1, i + 2);
+        forward(b, y, k, k + 1, 1, min(T, k + 1 + kNear));
+        const int i = k + 1;  // the helper's sum of row k + 1
+        if (i < T && i > kNear) {
+          wait_flags(done, fail, sy.s(i));
+          if (w == 0) b[i * NB + lane] += yv[(size_t)i * NB + lane];
         }
+      } else {
+        forward(b, y, k, k + 1, 1, T);
       }
       __syncthreads();
     }
@@ -570,77 +601,212 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
     return;
   }
 
-  if (w >= 4) return;  // the rest is four waves' work
   // ---- owners of tiles
-  const int o = (int)blockIdx.x - 2, ntiles = T * (T - 1) / 2 + max(0, T - 2);
-  if (ntiles > G - 2) {
-    // more tiles than workgroups: tiles o, o + (G - 2), .. each.  L_ik is formed
-    // once, by its owner, and the products read it from memory, so that a tile's
-    // task is the one product; within a phase the next columns come first.
-    const int H = G - 2;
-    int c0 = 0;  // the first tile of column k
-    for (int k = 0; k + 1 < T; ++k) {
-      const int c1 = c0 + T - 1 - k + (k >= 2 ? 1 : 0);
-      const int first = c0 + (k >= 2 ? 1 : 0);  // (past the diagonal tile)
-      bool have = false;
-      for (int t = o + max(0, first - o + H - 1) / H * H; t < c1; t += H) {
-        int i, j;
-        owner_tile(t, T, &i, &j);
-        if (!have) {
-          wait_flags(done, fail, sy.m(k));
-          load_inv(F, Mg + (size_t)k * kInvLen);
-          have = true;
-        }
-        double av[16];
-        load_rows(av, tile(S, i, k) + (size_t)16 * w * ld, ld);
-        lds_barrier();
-        dvec4 xt[4];
-        solve_rows(xt, av, F);
-        store_rows(xt, tile(Lf, i, k), ld);
-        publish(sy.l(i, k), done);
+  const int o = (int)blockIdx.x - 2;
+  if (many && o >= G - 2 - kForward) {
+    // the far terms of rows i = h, h + kForward, .. : L_ik y_k for k < i - kNear
+    const int h = o - (G - 2 - kForward);
+    lds_dbl* const b = (lds_dbl*)&sm.Y[0][0];
+    lds_dbl* const y = (lds_dbl*)sm.W;
+    for (int q = tid; q < (T + kForward - 1) / kForward * NB; q += 512) b[q] = 0.0;
+    for (int k = 0; k + kNear + 1 < T; ++k) {
+      const int lo = k + kNear + 1, i0 = lo + (h - lo % kForward + kForward) % kForward;
+      if (i0 >= T) break;
+      wait_flags(epoch + (ull)(k + 1), fail, sy.y());
+      if (tid < NB) y[tid] = xs[(size_t)k * NB + tid];
+      __syncthreads();
+      forward(b, y, k, i0, kForward, T);
+      __syncthreads();
+      if (i0 == lo) {  // its last
+        if (tid < NB) yv[(size_t)lo * NB + tid] = b[lo / kForward * NB + tid];
+        publish(sy.s(lo), done);
       }
-      // this phase's products: every flag they need first, a lane each
-      const int t1 = o + max(0, c1 - o + H - 1) / H * H;
+    }
+    if (w >= 4) return;
+  } else if (many) {
+    // more tiles than workgroups: tiles o, o + H, .. each, column by column, all eight
+    // waves on one tile at a time (wave w: rows 16 (w % 4) .., columns 32 (w / 4) ..).
+    // L_ik is formed once, by its owner, and the products read it from memory.  The
+    // tiles' chain from column to column (complete -> L -> flag -> product ->
+    // complete) has to keep up with workgroup 0's, so the next column's tile goes
+    // first, from the accumulators straight into its solve, with M_{k+1} fetched
+    // ahead of the product if it is there; the other products run while L is on
+    // its way.  The last kHeld tiles, which live longest, stay in registers: behind
+    // the acquire fences nothing stays in an L2, and reading and writing every
+    // tile in every phase (128 KB a product, 5.5 TB/s over the device) was what
+    // bound the first phases.  T = 43: 868 us without either and with four waves a
+    // tile, 834 with pairs of tiles a workgroup, 700 so.
+    const int H = G - 2 - kForward, half = w >> 2, wt = w & 3;
+    const int nown = o < ntiles ? (ntiles - o + H - 1) / H : 0, nmem = max(0, nown - kHeld);
+    auto own = [&](int q) {
+      int2 t;
+      owner_tile(o + q * H, T, &t.x, &t.y);
+      return t;
+    };
+    // 0: no product in phase k (the diagonal's last is workgroup 0's), 2: the last
+    auto product = [&](const int2& t, int k) {
+      const int last = t.x == t.y ? t.y - 2 : t.y - 1;
+      return k > last ? 0 : k == last ? 2 : 1;
+    };
+    int turn = 0;
+    auto buffer = [&](int n) { return n & 1 ? (lds_dbl*)sm.Y[0] : XF; };
+    auto multiply = [&](const int2& t, int k, dvec4 (&acc)[2], bool from_memory) {
+      double* const A = tile(S, t.x, t.y) + (size_t)16 * wt * ld + 32 * half;
+      double av[16];
+      dvec2 y[4];
+      const dvec2* const yp = (const dvec2*)(tile(Lf, t.y, k) + (size_t)(16 * wt + li) * ld + 32 * half + 4 * lk);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) y[q] = yp[8 * (q >> 1) + (q & 1)];
+      load_rows(av, tile(Lf, t.x, k) + (size_t)16 * wt * ld, ld);
+      if (from_memory) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[c][r] = A[(size_t)(4 * r + lk) * ld + 16 * c + li];
+      }
+      lds_dbl* const xt = buffer(turn++);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ((lds_dvec2*)xt)[(8 * wt + 4 * half + q) * 64 + lane] = y[q];
+      lds_barrier();
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        dvec2 f[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) f[c] = ((const lds_dvec2*)xt)[((2 * half + c) * 8 + m) * 64 + lane];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) acc[c] = mfma(-av[2 * m + q], f[c][q], acc[c]);
+      }
+      const bool last = product(t, k) == 2;
+      if (from_memory || last) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) A[(size_t)(4 * r + lk) * ld + 16 * c + li] = acc[c][r];
+      }
+      if (last) publish(sy.a(t.x, t.y), done);
+    };
+    auto load_m = [&](dvec2 (&mf)[3], int j) {
+      const dvec2* const M = (const dvec2*)(Mg + (size_t)j * kInvLen);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) mf[q] = M[min(tid + 512 * q, kInvFrag / 2 - 1)];
+    };
+    // L_ij of the complete tile in acc; mf: M_j's fragments if they are here already
+    auto solve = [&](const int2& t, dvec4 (&acc)[2], dvec2 (&mf)[3], bool have) {
+      lds_dbl* const rows = (lds_dbl*)sm.Y[1];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rows[(16 * wt + 4 * r + lk) * TS + 32 * half + 16 * c + li] = acc[c][r];
+      if (!have) {
+        wait_flags(done, fail, sy.m(t.y));
+        load_m(mf, t.y);
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        if (tid + 512 * q < kInvFrag / 2) ((lds_dvec2*)F)[tid + 512 * q] = mf[q];
+      lds_barrier();
+      // (the halves take column blocks 0, 3 and 1, 2: the same work)
+      double av[16];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        const dvec2 v = *(const lds_dvec2*)(rows + (16 * wt + li) * TS + 16 * (m >> 1) + 4 * lk + 2 * (m & 1));
+        av[2 * m] = v[0];
+        av[2 * m + 1] = v[1];
+      }
+      double* const L = tile(Lf, t.x, t.y);
+      auto blocks = [&](auto m0, auto m1) {
+        dvec4 xt;
+        solve_block<decltype(m0)::value>(xt, av, F);
+        dvec4 xu;
+        solve_block<decltype(m1)::value>(xu, av, F);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          L[(size_t)(16 * wt + li) * ld + 16 * decltype(m0)::value + 4 * r + lk] = xt[r];
+          L[(size_t)(16 * wt + li) * ld + 16 * decltype(m1)::value + 4 * r + lk] = xu[r];
+        }
+      };
+      if (half) blocks(std::integral_constant<int, 2>(), std::integral_constant<int, 1>());
+      else blocks(std::integral_constant<int, 3>(), std::integral_constant<int, 0>());
+      publish(sy.l(t.x, t.y), done);
+    };
+    // wave 0: the flags of phase k's products of own tiles q0 .. q1 - 1, a lane each
+    auto await_products = [&](int q0, int q1, int k) {
       if (tid < 64) {
-        for (int t = t1 + (tid >> 1) * H; t < ntiles; t += 32 * H) {
-          int i, j;
-          owner_tile(t, T, &i, &j);
-          if (!(i == j && k > j - 2)) poll(sy.l(tid & 1 ? j : i, k), done, fail);
+        for (int q = q0 + (tid >> 1); q < q1; q += 32) {
+          const int2 t = own(q);
+          if (product(t, k)) poll(sy.l(tid & 1 ? t.y : t.x, k), done, fail);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       }
       __syncthreads();
-      for (int t = t1; t < ntiles; t += H) {
-        int i, j;
-        owner_tile(t, T, &i, &j);
-        if (i == j && k > j - 2) continue;  // workgroup 0's product
-        dvec4 acc[4];
-        double av[16], bv[16];
-        load_rows(bv, tile(Lf, j, k) + (size_t)16 * w * ld, ld);
-        load_rows(av, tile(Lf, i, k) + (size_t)16 * w * ld, ld);
-        acc_load(acc, tile(S, i, j), ld);
-        dvec4 x[4], yt[4];
+    };
+    auto load_tile = [&](const int2& t, dvec4 (&acc)[2]) {
+      const double* const A = tile(S, t.x, t.y) + (size_t)16 * wt * ld + 32 * half;
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) yt[mb] = dvec4{bv[4 * mb], bv[4 * mb + 1], bv[4 * mb + 2], bv[4 * mb + 3]};
-        put_result(XF, w, yt);
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) x[mb] = dvec4{av[4 * mb], av[4 * mb + 1], av[4 * mb + 2], av[4 * mb + 3]};
-        lds_barrier();
-        acc_update(acc, x, XF);
-        acc_store(acc, tile(S, i, j), ld);
-        if (j == (i == j ? k + 2 : k + 1)) publish(sy.a(i, j), done);
-        else lds_barrier();
-      }
-      __syncthreads();
-      c0 = c1;
+        for (int r = 0; r < 4; ++r) acc[c][r] = A[(size_t)(4 * r + lk) * ld + 16 * c + li];
+    };
+    int2 held[kHeld];
+    dvec4 acc[kHeld][2];
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+      held[u] = nmem + u < nown ? own(nmem + u) : make_int2(0, 0);
+      load_tile(held[u], acc[u]);
     }
+    int cur = 0;  // own tiles of columns up to k
+    for (; cur < nown; ++cur) {
+      const int2 t = own(cur);
+      if (t.y != 0) break;
+      dvec2 mf[3];
+      dvec4 a0[2];
+      load_tile(t, a0);
+      solve(t, a0, mf, false);
+    }
+    auto column = [&](const int2& t, int k, dvec4 (&acc)[2], bool from_memory) {
+      dvec2 mf[3];
+      const bool have = *(lds_flag*)sm.prog != 0;
+      if (have) load_m(mf, k + 1);
+      multiply(t, k, acc, from_memory);
+      solve(t, acc, mf, have);
+    };
+    for (int k = 0; k + 1 < T; ++k) {
+      for (; cur < nown; ++cur) {
+        const int2 t = own(cur);
+        if (t.y != k + 1) break;
+        if (t.x == t.y) continue;
+        if (tid == 0) *(lds_flag*)sm.prog = peek(sy.m(k + 1)) >= done;
+        await_products(cur, cur + 1, k);
+        if (cur < nmem) {
+          dvec4 am[2];
+          column(t, k, am, true);
+        }
+#pragma unroll
+        for (int u = 0; u < kHeld; ++u)
+          if (cur == nmem + u) column(t, k, acc[u], false);
+      }
+      await_products(cur, nown, k);
+      for (int q = cur; q < nmem; ++q) {
+        dvec4 am[2];
+        const int2 t = own(q);
+        if (product(t, k)) multiply(t, k, am, true);
+      }
+#pragma unroll
+      for (int u = 0; u < kHeld; ++u)
+        if (nmem + u >= cur && nmem + u < nown && product(held[u], k)) multiply(held[u], k, acc[u], false);
+      __syncthreads();
+    }
+    if (w >= 4) return;
   } else {
+    if (w >= 4) return;  // one tile is four waves' work
     int i, j;
     owner_tile(o, T, &i, &j);
     double* const Aij = tile(S, i, j);
     const bool diag = i == j;
     dvec4 acc[4];
-    acc_load(acc, Aij, ld);
+    acc_load(acc, Aij, ld, w);
     const int steps = diag ? j - 1 : j;
     for (int k = 0; k < steps; ++k) {
       double av[16], bv[16];
@@ -663,7 +829,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
       lds_barrier();
     }
     if (j > 0 && !(diag && steps == 0)) {
-      acc_store(acc, Aij, ld);
+      acc_store(acc, Aij, ld, w);
       publish(sy.a(i, j), done);
     }
     if (!diag) {
@@ -687,7 +853,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
       lds_barrier();
       dvec4 xt[4];
       solve_rows(xt, av, F);
-      store_rows(xt, tile(Lf, i, j), ld);
+      store_rows(xt, tile(Lf, i, j), ld, w);
       publish(sy.l(i, j), done);
     }
   }
@@ -724,7 +890,7 @@ int launch_chol(psba_ctx* c) {
     // the diagonal chain, the triangular solves and, up to what is resident, a
     // workgroup for every other tile
     const int want = T == 1 ? 1 : 2 + T * (T - 1) / 2 + std::max(0, T - 2);
-    if (resident < std::min(want, 3)) return PSBA_ERR_UNSUPPORTED;
+    if (resident < std::min(want, 3 + kForward)) return PSBA_ERR_UNSUPPORTED;
     c->chol_grid = std::min(want, resident);
   }
   probe_begin(c, PSBA_PROBE_FACTOR);
@@ -737,7 +903,7 @@ int launch_chol(psba_ctx* c) {
   return PSBA_OK;
 }
 
-long chol_sync_words(int T) { return 2 + 2L * T + (long)T * (T + 1); }
+long chol_sync_words(int T) { return 3 + 3L * T + (long)T * (T + 1); }
 long chol_inv_len(int T) { return (long)T * kInvLen; }
 
 }  // namespace psba
