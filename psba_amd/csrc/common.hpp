@@ -237,6 +237,17 @@ __device__ inline bool gated_off(const unsigned char* run, const int* ownr, int 
   return run && !run[ownr ? ownr[i] : 0];
 }
 
+// acc += (src of lane Q of the 16-lane row) * mul, the broadcast inside the FMA.
+// Volatile: the order of such steps is the schedule, and it keeps
+// the two instructions that the hardware wants between a write of src and its
+// read by DPP.
+template <int Q>
+__device__ __forceinline__ void fmac_bcast(double& acc, double src, double mul) {
+  __asm__ volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                   : "+v"(acc)
+                   : "v"(src), "v"(mul), "n"(Q));
+}
+
 // Workgroups of a launch go to the 8 XCDs round-robin (workgroup b to XCD
 // b % 8), each XCD with its own L2.  A grid of xcd_grid(n) workgroups with
 // item = xcd_item(b, n) gives every XCD one contiguous eighth of an n-item

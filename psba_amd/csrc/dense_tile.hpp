@@ -59,17 +59,6 @@ __device__ __forceinline__ double fast_rsq(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// acc += (src of lane Q of the 16-lane row) * mul, the broadcast inside the FMA.
-// Volatile, as the steps around it: their order is the schedule, and it keeps
-// the two instructions that the hardware wants between a write of src and its
-// read by DPP.
-template <int Q>
-__device__ __forceinline__ void fmac_bcast(double& acc, double src, double mul) {
-  __asm__ volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-                   : "+v"(acc)
-                   : "v"(src), "v"(mul), "n"(Q));
-}
-
 // Elimination step C of a 16-column block: a is row l % 16 of the diagonal
 // block (the same in each 16-lane row of the wave), x this lane's row below it;
 // r = 1 / pivot.  Both lose column C times their multiplier (x[q] -= x[C] a_q[C] / pivot,

@@ -1,4 +1,4 @@
-// Reduced camera system of the plain FP64 path:
+// Reduced camera system:
 //   S_kl = delta_kl (U_k + mu I) - sum_{i in P(k,l)} W_ik V_i^-1 W_il^T   (k >= l)
 //   e_a,j = g_a,j - sum_i W_ij (V_i^-1 g_b,i)
 // Reference: PSBA/CL_files/compute_Yblks.cl, compute_S.cl, compute_ea.cl.
@@ -8,13 +8,27 @@
 // R is the storage and chunk-accumulation type (double on the plain path,
 // float on the mixed path); V^-1 is always FP64 and the chunk partials are
 // summed in FP64.
+#include <algorithm>
+#include <type_traits>
+
 #include "context.hpp"
 
-#ifndef PSBA_SCHUR_XCD
-#define PSBA_SCHUR_XCD 1
-#endif
-
 namespace psba {
+
+typedef double dvec2 __attribute__((ext_vector_type(2)));
+
+// v of lane Q of each quad (DPP quad_perm)
+template <int Q>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), Q * 0x55, 0xF, 0xF, true));
+}
+template <int Q>
+__device__ __forceinline__ double quad_lane(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, Q * 0x55, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), Q * 0x55, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
 
 // One workgroup per chunk (one camera pair, at most kPairChunk shared points).
 //   1. the chunk's item indices (W_a, W_b observation rows and the point) go to
@@ -49,12 +63,8 @@ __device__ __forceinline__ void schur_chunk(int wg, const int2* __restrict__ ite
   static_assert(G * C2 <= 2 * kPairChunk * REC, "group partials must fit the staging buffer");
   R* const sY = sBuf;
   R* const sW = sBuf + kPairChunk * REC;
-#if PSBA_SCHUR_XCD
   int b = xcd_item(wg, nchunk);  // one share of the launch order per XCD
   if (b < 0) return;
-#else
-  int b = wg;
-#endif
   const int t = threadIdx.x;
   int cnt;
   if constexpr (SLOTS) {
@@ -91,31 +101,39 @@ __device__ __forceinline__ void schur_chunk(int wg, const int2* __restrict__ ite
     if (it < cnt) {
       const R* wa = W + (size_t)sIdx[it] * REC;
       const R* wb = W + (size_t)sIdx[kPairChunk + it] * REC;
-      const double* vi = Vinv + (size_t)sIdx[2 * kPairChunk + it] * 6;
+      const dvec2* vi = (const dvec2*)(Vinv + (size_t)sIdx[2 * kPairChunk + it] * 6);
       // every load first and unconditional (a lane's rows and elements past
-      // the record are clamped to the last one and not stored), so that one
+      // the record are clamped to the last ones and not stored), so that one
       // wait covers them all: per-lane loop bounds made each remainder a
-      // round of its own
-      constexpr int NR = (CNP + 3) / 4, NW = (REC + 3) / 4;
-      double v[6];
-      R wv[NR][3], bv[NW];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) v[k] = vi[k];
+      // round of its own.  The loads' number counts (a wave's load of 64 separate
+      // places takes the vector cache 16 cycles whatever its width): W_b in
+      // 16-byte pieces and a third of V^-1 a lane, passed round the quad, instead
+      // of single values and all of V^-1 (6 parameters, float: 5 loads for 10;
+      // 512 windows' chunks 635 -> 424 us)
+      constexpr int VEC = 16 / (int)sizeof(R);
+      typedef R Vec __attribute__((ext_vector_type(VEC), aligned(sizeof(R))));
+      constexpr int NR = (CNP + 3) / 4, NW = ((REC + VEC - 1) / VEC + 3) / 4;
+      R wv[NR][3];
+      Vec bv[NW];
+      dvec2 v = vi[min(q, 2)];
 #pragma unroll
       for (int j = 0; j < NR; ++j) {
         const int r = min(q + 4 * j, CNP - 1);
 #pragma unroll
         for (int c = 0; c < 3; ++c) wv[j][c] = wa[3 * r + c];
       }
+      auto at = [&](int j) { return min(VEC * (q + 4 * j), REC - VEC); };
 #pragma unroll
-      for (int j = 0; j < NW; ++j) bv[j] = wb[min(q + 4 * j, REC - 1)];
+      for (int j = 0; j < NW; ++j) bv[j] = *(const Vec*)(wb + at(j));
       // (the empty asm keeps the compiler from sinking the loads of a row
       // used under a condition into that condition's block)
 #pragma unroll
       for (int j = 0; j < NR; ++j)
 #pragma unroll
         for (int c = 0; c < 3; ++c) __asm__ volatile("" : "+v"(wv[j][c]));
-      const R v00 = (R)v[0], v01 = (R)v[1], v02 = (R)v[2], v11 = (R)v[3], v12 = (R)v[4], v22 = (R)v[5];
+      const R lo = (R)v[0], hi = (R)v[1];
+      const R v00 = quad_lane<0>(lo), v01 = quad_lane<0>(hi), v02 = quad_lane<1>(lo), v11 = quad_lane<1>(hi),
+              v12 = quad_lane<2>(lo), v22 = quad_lane<2>(hi);
 #pragma unroll
       for (int j = 0; j < NR; ++j) {
         const int r = q + 4 * j;
@@ -129,7 +147,10 @@ __device__ __forceinline__ void schur_chunk(int wg, const int2* __restrict__ ite
       }
 #pragma unroll
       for (int j = 0; j < NW; ++j)
-        if (q + 4 * j < REC) sW[it * REC + q + 4 * j] = bv[j];
+        if (VEC * (q + 4 * j) < REC) {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) sW[it * REC + at(j) + k] = bv[j][k];
+        }
     }
   }
   __syncthreads();
@@ -194,7 +215,8 @@ __global__ __launch_bounds__(256) void k_schur_chunks(const int2* __restrict__ i
 }
 
 // one block per lower block position (k >= l) of S, including empty ones
-// Blocks [0, nlb) write the lower block positions; the remaining blocks
+// Blocks [0, nlb) write the lower block positions (a pair's partials lie at its
+// chunks 0, cpg, 2 cpg, ..); the remaining blocks
 // rewrite the padding rows n..n_pad-1 as identity rows (a failed
 // factorisation may have left anything there).
 template <int CNP, typename R>
@@ -202,7 +224,7 @@ __device__ __forceinline__ void schur_finish_block(int b, const int* __restrict_
                                                    const int* __restrict__ psp, const R* __restrict__ part,
                                                    const double* __restrict__ U, const unsigned char* __restrict__ fix,
                                                    double mu, const double* __restrict__ mu_p, int ld, int nlb, int n,
-                                                   double* __restrict__ S) {
+                                                   int cpg, double* __restrict__ S) {
   constexpr int C2 = CNP * CNP;
   if (mu_p) mu = *mu_p;
   if (b >= nlb) {
@@ -218,7 +240,11 @@ __device__ __forceinline__ void schur_finish_block(int b, const int* __restrict_
   for (int t = threadIdx.x; t < C2; t += blockDim.x) {
     const int r = t / CNP, cc = t - r * CNP;
     double acc = 0.0;
-    if (q >= 0) acc = ordered_sum<16>(psp[q], psp[q + 1], [&](int h) { return (double)part[(size_t)h * C2 + t]; });
+    if (q >= 0) {
+      const int h0 = psp[q];
+      acc = ordered_sum<16>(0, (psp[q + 1] - h0 + cpg - 1) / cpg,
+                            [&](int h) { return (double)part[(size_t)(h0 + h * cpg) * C2 + t]; });
+    }
     double val;
     if (k == l) {
       double u = U[(size_t)k * C2 + t];
@@ -297,17 +323,28 @@ __global__ __launch_bounds__(256) void k_ea_chunks(const int* __restrict__ cam_o
   ea_chunk<CNP, R>(blockIdx.x, cam_obs, cb, ce, obs_pt, W, z, part, ownr, run, rec, sP, sO, sI);
 }
 
-// One problem's Schur chunks and e_a chunks in one launch (they share no
-// data).  The launch is in groups of eight workgroups (one per XCD); of every
+// One problem's Schur work and e_a chunks in one launch (they share no data).
+// The launch is in groups of eight workgroups (one per XCD); of every
 // period + 1 groups, the first `period` are Schur groups and the last an e_a
 // group, until the e_a groups (neg) are placed, then Schur groups only.  A
 // Schur group gs gives workgroup index 8 gs + blockIdx % 8, the index
-// k_schur_chunks' workgroup on the same XCD has (SLOTS form, so the same XCD
-// shares of the launch order); e_a group eg takes camera chunk
-// 8 eg + blockIdx % 8.  The memory-streaming e_a chunks so run beside the
-// latency-bound Schur chunks.  The e_a chunks take their LDS from the Schur
-// staging buffer.  Each chunk's arithmetic is its own kernel's, so the
-// partials are the same bits.
+// k_schur_chunks' workgroup on the same XCD has (so the same XCD shares of the
+// launch order); e_a group eg takes camera chunk 8 eg + blockIdx % 8.  The
+// memory-streaming e_a chunks so run beside the Schur work.
+struct LaunchSlot {
+  int schur = -1, ea = -1;
+  __device__ __forceinline__ LaunchSlot(int block, int neg, int period) {
+    const int g = block >> 3, l8 = block & 7;
+    const int q = g / (period + 1), rm = g - q * (period + 1);
+    if (q >= neg) schur = 8 * (neg * period + (g - neg * (period + 1))) + l8;
+    else if (rm == period) ea = 8 * q + l8;
+    else schur = 8 * (q * period + rm) + l8;
+  }
+};
+
+// (Mixed precision.)  The e_a chunks take their LDS from the Schur staging
+// buffer.  Each chunk's arithmetic is its own kernel's, so the partials are the
+// same bits.
 template <int CNP, typename R>
 __global__ __launch_bounds__(256) void k_schur_ea_chunks(const R* __restrict__ W, const double* __restrict__ Vinv,
                                                          R* __restrict__ spart, int nchunk,
@@ -321,25 +358,157 @@ __global__ __launch_bounds__(256) void k_schur_ea_chunks(const R* __restrict__ W
   __shared__ R sBuf[2 * kPairChunk * 3 * CNP];
   __shared__ int sIdx[3 * kPairChunk];
   __shared__ int sMeta[2];
-  const int g = (int)blockIdx.x >> 3, l8 = (int)blockIdx.x & 7;
-  const int q = g / (period + 1), rm = g - q * (period + 1);
-  int gs = -1, eg = -1;
-  if (q < neg) {
-    if (rm == period) eg = q;
-    else gs = q * period + rm;
-  } else {
-    gs = neg * period + (g - neg * (period + 1));
-  }
-  if (gs >= 0) {
-    const int wg = 8 * gs + l8;
-    if (wg >= nb_schur) return;
-    schur_chunk<CNP, R, true>(wg, nullptr, nullptr, nullptr, nullptr, W, Vinv, spart, nullptr, nullptr, nchunk,
+  const LaunchSlot ls(blockIdx.x, neg, period);
+  if (ls.schur >= 0) {
+    if (ls.schur >= nb_schur) return;
+    schur_chunk<CNP, R, true>(ls.schur, nullptr, nullptr, nullptr, nullptr, W, Vinv, spart, nullptr, nullptr, nchunk,
                               nullptr, rec, sBuf, sIdx, sMeta);
   } else {
-    const int b = 8 * eg + l8;
-    if (b >= ncc) return;
+    if (ls.ea >= ncc) return;
     int* const sO = (int*)(sBuf + CH * CNP);
-    ea_chunk<CNP, R>(b, nullptr, cb, ce, nullptr, W, z, epart, nullptr, nullptr, erec, sBuf, sO, sO + CH);
+    ea_chunk<CNP, R>(ls.ea, nullptr, cb, ce, nullptr, W, z, epart, nullptr, nullptr, erec, sBuf, sO, sO + CH);
+  }
+}
+
+// The FP64 Schur products of one problem, without LDS: a wave takes a group (up to
+// c->schur_group consecutive chunks of one camera pair) four items at a time, one
+// in each 16-lane row.  Lane l < CNP of a row has row l of W_a and of W_b (and
+// element l < 6 of V^-1); it forms row l of Y = W_a V^-1 and column l of Y W_b^T,
+// with what other lanes hold broadcast inside the multiply-adds (fmac_bcast).
+// The four rows' sums meet at the end of the group.
+//
+// Bound by the rows' lines on their way from L2 to the L1s (an item's two rows
+// and V^-1: 7 lines of 128 B at 9 parameters, 14 TB/s): so nothing else may take
+// long.  A pass's rows are under way while the one before is multiplied.  Staging
+// 64 items in LDS for 3 x 3 register blocks (schur_chunk, which mixed precision
+// keeps for its order of sums, and 6 parameters, where a row has only six lanes'
+// work) took LDS bandwidth and four barriers a chunk, and as long to sum its
+// group partials as to form them: 88 cameras with 9 parameters 246 -> 214 us
+// a launch with the e_a chunks, 300 with 9 314 -> 230, 54 with 11 18.5 -> 13.8, 30
+// with 16 18.6 -> 13.9; with 6 parameters it would be 51 -> 70 (138 cameras).
+typedef const __attribute__((address_space(1))) double glb_dbl;  // (a pointer that went through a shuffle)
+
+template <int CNP>
+struct SchurPass {
+  double a[3], b[3], v;
+  __device__ __forceinline__ void load(glb_dbl* wa, glb_dbl* wb, glb_dbl* vi) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) a[k] = wa[k];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) b[k] = wb[k];
+    v = *vi;
+  }
+  template <int R, int K>
+  __device__ __forceinline__ static void outer(double (&acc)[CNP], double y, double bk) {
+    if constexpr (R < CNP) {
+      fmac_bcast<R>(acc[R], y, bk);
+      outer<R + 1, K>(acc, y, bk);
+    }
+  }
+  __device__ __forceinline__ void multiply(double (&acc)[CNP]) {
+    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+    __asm__ volatile("s_nop 1" : "+v"(v));  // (a copy of v may lie just before)
+    fmac_bcast<0>(y0, v, a[0]);
+    fmac_bcast<1>(y1, v, a[0]);
+    fmac_bcast<2>(y2, v, a[0]);
+    fmac_bcast<1>(y0, v, a[1]);
+    fmac_bcast<3>(y1, v, a[1]);
+    fmac_bcast<4>(y2, v, a[1]);
+    fmac_bcast<2>(y0, v, a[2]);
+    fmac_bcast<4>(y1, v, a[2]);
+    fmac_bcast<5>(y2, v, a[2]);
+    outer<0, 0>(acc, y0, b[0]);
+    outer<0, 1>(acc, y1, b[1]);
+    outer<0, 2>(acc, y2, b[2]);
+  }
+};
+
+template <int CNP>
+__device__ __forceinline__ void schur_group(const int4 grp, const int4* __restrict__ rec,
+                                            const double* __restrict__ W, const double* __restrict__ Vinv,
+                                            double* __restrict__ part) {
+  constexpr int REC = 3 * CNP, B = 1;  // passes loaded together
+  const int lane = threadIdx.x & 63, row = lane >> 4, l = lane & 15;
+  const int n = grp.y - grp.x, np = (n + 3) >> 2;
+  // sixteen passes' items, one a lane (lane 16 row + l: pass l's item of the row);
+  // past the end the last one, not counted
+  const int4* const r0 = rec + grp.x;
+  auto item = [&](int p0) { return r0[min(4 * (p0 + l) + row, n - 1)]; };
+  struct At { const double *wa, *wb, *vi; };
+  auto at_of = [&](const int4& r) { return At{W + (size_t)r.x * REC, W + (size_t)r.y * REC, Vinv + (size_t)r.z * 6}; };
+  int4 ahead = item(0);
+  At at = at_of(ahead);
+  ahead = item(16);
+  const int off = 3 * min(l, CNP - 1), voff = min(l, 5);
+  auto of_pass = [&](const double* x, int p) {
+    return (glb_dbl*)__shfl((unsigned long long)x, (lane & 48) + (p & 15), 64);
+  };
+  auto load = [&](SchurPass<CNP> (&ps)[B], int p) {
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      ps[u].load(of_pass(at.wa, p + u) + off, of_pass(at.wb, p + u) + off, of_pass(at.vi, p + u) + voff);
+    __asm__ volatile("" ::: "memory");  // the loads go out ahead of what follows
+  };
+  double acc[CNP];
+#pragma unroll
+  for (int r = 0; r < CNP; ++r) acc[r] = 0.0;
+  auto multiply = [&](SchurPass<CNP> (&ps)[B], int p) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      if (4 * (p + u + 1) > n) {
+        const bool on = 4 * (p + u) + row < n;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) ps[u].b[k] = on ? ps[u].b[k] : 0.0;
+      }
+      ps[u].multiply(acc);
+    }
+  };
+  SchurPass<CNP> x[B], y[B];
+  load(x, 0);
+#pragma unroll 1
+  for (int p = 0; p < np; p += 2 * B) {
+    load(y, p + B);
+    multiply(x, p);
+    if (((p + 2 * B) & 15) == 0) {
+      at = at_of(ahead);
+      ahead = item(p + 2 * B + 16);
+    }
+    load(x, p + 2 * B);
+    if (p + B < np) multiply(y, p + B);
+  }
+  double* const out = part + (size_t)grp.z * (CNP * CNP);
+#pragma unroll
+  for (int r = 0; r < CNP; ++r) {
+    double t = acc[r];
+    t += __shfl_xor(t, 16, 64);
+    t += __shfl_xor(t, 32, 64);
+    if (lane < CNP) out[r * CNP + lane] = t;
+  }
+}
+
+// One problem's Schur groups and e_a chunks in one launch, as k_schur_ea_chunks
+// has them; a Schur workgroup's four waves take four neighbouring groups
+template <int CNP>
+__global__ __launch_bounds__(256) void k_schur_ea_groups(const double* __restrict__ W,
+                                                         const double* __restrict__ Vinv,
+                                                         double* __restrict__ spart, int ngroup,
+                                                         const int4* __restrict__ grp, const int4* __restrict__ rec,
+                                                         int nb_schur, int neg, int period, int ncc,
+                                                         const int* __restrict__ cb, const int* __restrict__ ce,
+                                                         const double* __restrict__ z, double* __restrict__ epart,
+                                                         const int2* __restrict__ erec) {
+  constexpr int CH = ea_chunk_obs<CNP>();
+  __shared__ double sP[CH * CNP];
+  __shared__ int sO[CH], sI[CH];
+  const LaunchSlot ls(blockIdx.x, neg, period);
+  if (ls.schur >= 0) {
+    if (ls.schur >= nb_schur) return;
+    const int wg = xcd_item(ls.schur, (ngroup + 3) >> 2);
+    const int g = 4 * wg + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (wg < 0 || g >= ngroup) return;
+    schur_group<CNP>(grp[g], rec, W, Vinv, spart);
+  } else if (ls.ea < ncc) {
+    ea_chunk<CNP, double>(ls.ea, nullptr, cb, ce, nullptr, W, z, epart, nullptr, nullptr, erec, sP, sO, sI);
   }
 }
 
@@ -370,12 +539,12 @@ __global__ __launch_bounds__(256) void k_schur_ea_finish(const int* __restrict__
                                                          const int* __restrict__ psp, const R* __restrict__ spart,
                                                          const double* __restrict__ U,
                                                          const unsigned char* __restrict__ fix,
-                                                         const double* __restrict__ mu_p, int ld, int nlb, int n,
+                                                         const double* __restrict__ mu_p, int ld, int nlb, int n, int cpg,
                                                          double* __restrict__ S, int nfin, const int* __restrict__ ccp,
                                                          const R* __restrict__ epart, const double* __restrict__ ga,
                                                          int nc, double* __restrict__ ea, double mu) {
   if ((int)blockIdx.x < nfin)
-    schur_finish_block<CNP, R>(blockIdx.x, lblock_pair, psp, spart, U, fix, mu, mu_p, ld, nlb, n, S);
+    schur_finish_block<CNP, R>(blockIdx.x, lblock_pair, psp, spart, U, fix, mu, mu_p, ld, nlb, n, cpg, S);
   else
     ea_finish_one<CNP, R>(((int)blockIdx.x - nfin) * blockDim.x + threadIdx.x, ccp, epart, ga, nc, ea, nullptr,
                           nullptr);
@@ -383,10 +552,12 @@ __global__ __launch_bounds__(256) void k_schur_ea_finish(const int* __restrict__
 
 template <int CNP, typename R>
 static void run_schur_t(psba_ctx* c, double mu, const R* W, R* schpart, R* eapart) {
-  // the Schur and e_a chunks in one launch (the e_a chunks after the Schur
-  // chunks, so they fill the CUs that the Schur launch's tail leaves idle),
-  // then both finishes in one launch
-  const int nb_schur = c->n_schunk > 0 ? (int)(PSBA_SCHUR_XCD ? xcd_grid(c->n_schunk) : c->n_schunk) : 0;
+  // the Schur work and the e_a chunks in one launch (the e_a chunks after the
+  // first Schur workgroups, so they fill the CUs that the Schur launch's tail
+  // leaves idle), then both finishes in one launch
+  constexpr bool kGroups = std::is_same<R, double>::value && CNP > 6;
+  const int nwork = kGroups ? (c->n_sgroup + 3) / 4 : c->n_schunk;
+  const int nb_schur = nwork > 0 ? (int)xcd_grid(nwork) : 0;
   const int nsg = (nb_schur + 7) / 8, neg = (c->n_cchunk + 7) / 8;
   if (nsg + neg > 0) {
     // (with fewer Schur groups than e_a groups, period 1 and the surplus
@@ -394,15 +565,21 @@ static void run_schur_t(psba_ctx* c, double mu, const R* W, R* schpart, R* eapar
     const int period = neg > 0 ? std::max(1, nsg / neg) : 1;
     const int ngroups = neg * (period + 1) + std::max(0, nsg - neg * period);
     probe_begin(c, PSBA_PROBE_SCHUR);
-    hipLaunchKernelGGL((k_schur_ea_chunks<CNP, R>), dim3(8 * ngroups), dim3(256), 0, c->stream, W, c->Vinv,
-                       schpart, c->n_schunk, (const int4*)c->slot_items, nb_schur, neg, period, c->n_cchunk,
-                       c->cchunk_begin, c->cchunk_end, c->z, eapart, (const int2*)c->cchunk_rec);
+    if constexpr (kGroups)
+      hipLaunchKernelGGL((k_schur_ea_groups<CNP>), dim3(8 * ngroups), dim3(256), 0, c->stream, W, c->Vinv, schpart,
+                         c->n_sgroup, (const int4*)c->sgroup, (const int4*)c->item_rec, nb_schur, neg, period,
+                         c->n_cchunk, c->cchunk_begin, c->cchunk_end, c->z, eapart, (const int2*)c->cchunk_rec);
+    else
+      hipLaunchKernelGGL((k_schur_ea_chunks<CNP, R>), dim3(8 * ngroups), dim3(256), 0, c->stream, W, c->Vinv,
+                         schpart, c->n_schunk, (const int4*)c->slot_items, nb_schur, neg, period, c->n_cchunk,
+                         c->cchunk_begin, c->cchunk_end, c->z, eapart, (const int2*)c->cchunk_rec);
     probe_end(c, PSBA_PROBE_SCHUR);
   }
   const int nfin = c->n_lblocks + (c->n_pad - c->n), bs = CNP * CNP > 128 ? 256 : 128;
   hipLaunchKernelGGL((k_schur_ea_finish<CNP, R>), dim3(nfin + ceil_div((long)c->nc * CNP, bs)), dim3(bs), 0,
                      c->stream, c->lblock_pair, c->pair_schunk_ptr, schpart, c->U, c->fix, mu_of(c), c->n_pad,
-                     c->n_lblocks, c->n, c->S, nfin, c->cam_cchunk_ptr, eapart, c->g, c->nc, c->ea, mu);
+                     c->n_lblocks, c->n, kGroups ? c->schur_group : 1, c->S, nfin, c->cam_cchunk_ptr, eapart, c->g,
+                     c->nc, c->ea, mu);
 }
 
 template <int CNP>
@@ -516,7 +693,7 @@ static void run_b_schur_t(psba_batch* b) {
   const R* W = (const R*)b->W;
   R *schpart = (R*)b->schpart, *eapart = (R*)b->eapart;
   if (b->n_schunk > 0)
-    hipLaunchKernelGGL((k_schur_chunks<CNP, R, false>), dim3(PSBA_SCHUR_XCD ? xcd_grid(b->n_schunk) : b->n_schunk),
+    hipLaunchKernelGGL((k_schur_chunks<CNP, R, false>), dim3(xcd_grid(b->n_schunk)),
                        dim3(256), 0, b->stream, b->items, b->schunk_b, b->schunk_e, b->obs_pt, W, b->Vinv, schpart,
                        b->schunk_prob, b->active, b->n_schunk, (const int*)nullptr, (const int4*)nullptr);
   if (b->nlb > 0)

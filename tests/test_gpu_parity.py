@@ -62,6 +62,26 @@ def test_stages_match_oracle(P, O, gpu, config, kw):
     assert rel(g.buffer("EB"), o.buffer("EB")) < 1e-11
 
 
+# pairs of a few items, of several chunks; groups of one, two (10000 chunks and more)
+# and four chunks (20000), the last of a pair short
+@pytest.mark.parametrize("config,kw", [(1, dict(n_cams=3, n_pts=7)), (1, dict(cnp=16, n_cams=4, n_pts=90)),
+                                       (2, dict(n_cams=6, n_pts=1000)), (2, dict(n_cams=150, n_pts=9000)),
+                                       (2, dict(n_cams=150, n_pts=30000))])
+def test_schur_groups_match_oracle(P, O, gpu, config, kw):
+    sc = P.Scene(config, 11, **kw)
+    g, o = pair(P, O, sc)
+    O.set_threads(16)
+    g.jacobian_normal(1.0, 1.0)
+    o.jacobian_normal(1.0, 1.0)
+    mu = 1e-3 * o.max_uvdiag()
+    g.schur(mu)
+    o.schur(mu)
+    n = sc.cnp * sc.n_cams
+    tl = np.tril_indices(n)
+    assert rel(g.buffer("EA"), o.buffer("EA")) < 1e-11
+    assert rel(g.buffer("S").reshape(n, n)[tl], o.buffer("S").reshape(n, n)[tl]) < 1e-11
+
+
 def test_schur_is_deterministic(P, gpu):
     sc = P.Scene(2, 7, n_pts=4000, n_cams=24)
     a = P.Context.from_scene(sc)
