@@ -497,6 +497,18 @@ int build_schur_slots(psba_ctx* c) {
 // Points by descending track length, ties in ascending id (a stable radix
 // sort).  The back substitution takes its points in this order, so that the
 // points one wave handles in lockstep have tracks of similar length.
+// how many of the points, in that order, have tracks of at least kLongTrack
+__global__ void k_long_tracks(const int* __restrict__ order, const int* __restrict__ pt_ptr, int np,
+                              int* __restrict__ n) {
+  int lo = 0, hi = np;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1, i = order[mid];
+    if (pt_ptr[i + 1] - pt_ptr[i] >= kLongTrack) lo = mid + 1;
+    else hi = mid;
+  }
+  *n = lo;
+}
+
 int build_point_order(psba_ctx* c) {
   const int np = c->np;
   hipStream_t st = c->stream;
@@ -511,7 +523,9 @@ int build_point_order(psba_ctx* c) {
   Scratch tmp;
   PSBA_TRY(tmp.ensure(tb));
   IX_TRY(rocprim::radix_sort_pairs(tmp.p, tb, key.p, key_s.p, val.p, c->pt_order, (size_t)np, 0, 32, st));
+  hipLaunchKernelGGL(k_long_tracks, dim3(1), dim3(1), 0, st, c->pt_order, c->pt_ptr, np, val.p);
   IX_TRY(hipGetLastError());
+  IX_TRY(hipMemcpyAsync(&c->n_long, val.p, sizeof(int), hipMemcpyDeviceToHost, st));
   IX_TRY(hipStreamSynchronize(st));  // the temporaries are freed on return
   return PSBA_OK;
 }

@@ -651,6 +651,16 @@ int launch_vinv(psba_ctx* c, double mu) {
 constexpr int kBacksubPtsPerWave = 21;
 constexpr int kBacksubLdsDpa = 4096;  // camera parameters that go through LDS (32 KB)
 
+// Points of long tracks (kLongTrack observations and more, first in `order`) get
+// seven times the lanes, three points a wave: each triple of lanes sums every
+// seventh observation, and the seven sums are added in order.  Otherwise the
+// longest track's chain of loads bounds the launch (0.37 us a step): 300 cameras
+// with 9 parameters, longest track 300: 112 -> 28 us; 88 cameras: 44 -> 21; 138
+// cameras with 6: 40 -> 13; 30 with 16, longest track 20: 20 -> 11.  The line: an
+// observation for every triple; at 10, 16 and 24 the 88 cameras take 23, 23 and 25 us, the 30
+// cameras 14, 20 and 20, the 300 27, 27 and 26.
+constexpr int kLongLanes = 7;
+
 // With LDS_DPA the camera step dp[0..n) is first copied into LDS (dynamic
 // shared memory of n doubles), so that a long track waits for the W rows only.
 // SORTED: `order` holds the points by descending track length.
@@ -660,20 +670,30 @@ __global__ __launch_bounds__(256) void k_backsub(const int* __restrict__ pt_ptr,
                                                  const double* __restrict__ gb, int np, int n,
                                                  double* __restrict__ dp, double* __restrict__ eb,
                                                  const int* __restrict__ ownr, const unsigned char* __restrict__ run,
-                                                 const int* __restrict__ order) {
+                                                 const int* __restrict__ order, int n_long) {
   extern __shared__ double sDa[];
   if constexpr (LDS_DPA) {
     for (int q = threadIdx.x; q < n; q += blockDim.x) sDa[q] = dp[q];
     __syncthreads();
   }
   const int lane = threadIdx.x & 63;
-  const int grp = lane / 3;
-  const int cc = lane - 3 * grp;
+  const int cc = lane % 3;
   // slot -> point: with `order` (points by descending track length) the
   // points of a wave, which step through their observations together, have
   // tracks of similar length
-  const int slot = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * kBacksubPtsPerWave + grp;
-  const bool in = grp < kBacksubPtsPerWave && slot < np;
+  int grp = lane / 3, slot = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), part = 0, parts = 1;
+  bool in = grp < kBacksubPtsPerWave;
+  const int long_waves = SORTED ? (n_long + 2) / 3 : 0;
+  if (slot < long_waves) {
+    part = grp % kLongLanes;
+    parts = kLongLanes;
+    grp /= kLongLanes;
+    slot = 3 * slot + grp;
+    in = in && slot < n_long;
+  } else {
+    slot = (SORTED ? n_long : 0) + (slot - long_waves) * kBacksubPtsPerWave + grp;
+    in = in && slot < np;
+  }
   const int i = (in && SORTED) ? order[slot] : slot;
   const bool ok = in && (!run || run[ownr[i]]);
   R s = 0;
@@ -707,14 +727,16 @@ __global__ __launch_bounds__(256) void k_backsub(const int* __restrict__ pt_ptr,
     // (unconditional loads, so the waits count exactly), and the running sum
     // keeps its order.
     constexpr int PF = 2;
-    const int beg = ok ? pt_ptr[i] : 0, len = ok ? pt_ptr[i + 1] - beg : 0;
+    const int beg0 = ok ? pt_ptr[i] : 0, len0 = ok ? pt_ptr[i + 1] - beg0 : 0;
+    // this lane's share: observations beg, beg + parts, ..
+    const int beg = beg0 + min(part, max(0, len0 - 1)), len = max(0, (len0 - part + parts - 1) / parts);
     int lmax = len;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) lmax = max(lmax, __shfl_xor(lmax, off, 64));
     R wb[PF][CNP];
     int cb[PF];
     auto fetch = [&](int u, int st) {
-      const int o = beg + max(0, min(st, len - 1));
+      const int o = beg + parts * max(0, min(st, len - 1));
       cb[u] = obs_cam[o];
       const R* w = W + (size_t)o * 3 * CNP + cc;
 #pragma unroll
@@ -739,10 +761,16 @@ __global__ __launch_bounds__(256) void k_backsub(const int* __restrict__ pt_ptr,
       }
     }
   }
+  const int base = 3 * grp * parts;
+  if (SORTED && parts > 1) {
+    R t = 0;
+#pragma unroll
+    for (int u = 0; u < kLongLanes; ++u) t += __shfl(s, base + 3 * u + cc);
+    s = t;
+  }
   const double e = ok ? gb[3 * (size_t)i + cc] - (double)s : 0.0;
-  const int base = 3 * grp;
   const double e0 = __shfl(e, base), e1 = __shfl(e, base + 1), e2 = __shfl(e, base + 2);
-  if (!ok) return;
+  if (!ok || part != 0) return;
   eb[3 * (size_t)i + cc] = e;
   // row cc of the symmetric 3x3 from its packed entries (0 1 2 / 1 3 4 / 2 4 5)
   const double* v = Vinv + (size_t)i * 6;
@@ -753,13 +781,13 @@ __global__ __launch_bounds__(256) void k_backsub(const int* __restrict__ pt_ptr,
 template <int CNP, typename R>
 static void backsub_launch(hipStream_t st, const int* pt_ptr, const int* obs_cam, const R* W, const double* Vinv,
                            const double* gb, int np, int n, double* dp, double* eb, const int* pt_ownr,
-                           const unsigned char* run, int block, const int* order = nullptr) {
-  const int per_block = (block / 64) * kBacksubPtsPerWave;
+                           const unsigned char* run, int block, const int* order = nullptr, int n_long = 0) {
+  const long waves = ceil_div(n_long, 3) + ceil_div(np - n_long, kBacksubPtsPerWave);
   const size_t lds = n <= kBacksubLdsDpa ? sizeof(double) * (size_t)n : 0;
   auto kern = n <= kBacksubLdsDpa ? (order ? k_backsub<CNP, R, true, true> : k_backsub<CNP, R, true, false>)
                                   : (order ? k_backsub<CNP, R, false, true> : k_backsub<CNP, R, false, false>);
-  hipLaunchKernelGGL(kern, dim3(ceil_div(np, per_block)), dim3(block), lds, st, pt_ptr, obs_cam, W, Vinv, gb, np, n,
-                     dp, eb, pt_ownr, run, order);
+  hipLaunchKernelGGL(kern, dim3(ceil_div(waves, block / 64)), dim3(block), lds, st, pt_ptr, obs_cam, W, Vinv, gb, np,
+                     n, dp, eb, pt_ownr, run, order, n_long);
 }
 
 template <int CNP>
@@ -770,7 +798,7 @@ static void run_backsub(psba_ctx* c) {
     // 33 against 64-71 us at the 88-camera scene)
     backsub_launch<CNP, float>(c->stream, c->pt_ptr, c->obs_cam, c->W32, c->Vinv, c->g + c->n, c->np, c->n, c->dp, c->eb, (const int*)nullptr, (const unsigned char*)nullptr, 256);
   else
-    backsub_launch<CNP, double>(c->stream, c->pt_ptr, c->obs_cam, c->W, c->Vinv, c->g + c->n, c->np, c->n, c->dp, c->eb, (const int*)nullptr, (const unsigned char*)nullptr, 256, c->pt_order);
+    backsub_launch<CNP, double>(c->stream, c->pt_ptr, c->obs_cam, c->W, c->Vinv, c->g + c->n, c->np, c->n, c->dp, c->eb, (const int*)nullptr, (const unsigned char*)nullptr, 256, c->pt_order, c->n_long);
   probe_end(c, PSBA_PROBE_BSOLVE);
 }
 
@@ -1178,7 +1206,7 @@ static void run_backsub_rhs(psba_ctx* c, const double* gb, double* dp_out) {
   if (c->mixed())
     backsub_launch<CNP, float>(c->stream, c->pt_ptr, c->obs_cam, c->W32, c->Vinv, gb, c->np, c->n, dp_out, c->eb, (const int*)nullptr, (const unsigned char*)nullptr, 256);
   else
-    backsub_launch<CNP, double>(c->stream, c->pt_ptr, c->obs_cam, c->W, c->Vinv, gb, c->np, c->n, dp_out, c->eb, (const int*)nullptr, (const unsigned char*)nullptr, 256, c->pt_order);
+    backsub_launch<CNP, double>(c->stream, c->pt_ptr, c->obs_cam, c->W, c->Vinv, gb, c->np, c->n, dp_out, c->eb, (const int*)nullptr, (const unsigned char*)nullptr, 256, c->pt_order, c->n_long);
 }
 
 int launch_backsub_rhs(psba_ctx* c, const double* gb, double* dp_out) {

@@ -82,6 +82,27 @@ def test_schur_groups_match_oracle(P, O, gpu, config, kw):
     assert rel(g.buffer("S").reshape(n, n)[tl], o.buffer("S").reshape(n, n)[tl]) < 1e-11
 
 
+# long tracks by seven lane triples: none, few and many of them, lengths around seven
+# and its multiples, three points to a wave
+@pytest.mark.parametrize("config,kw", [(1, dict(n_cams=4, n_pts=50)), (1, dict(n_cams=9, n_pts=30)),
+                                       (2, dict(n_cams=60, n_pts=700)), (2, dict(n_cams=150, n_pts=9000)),
+                                       (1, dict(cnp=16, n_cams=24, n_pts=400))])
+def test_backsub_of_long_tracks(P, O, gpu, config, kw):
+    sc = P.Scene(config, 12, **kw)
+    g, o = pair(P, O, sc)
+    O.set_threads(16)
+    g.jacobian_normal(1.0, 1.0)
+    o.jacobian_normal(1.0, 1.0)
+    mu = 1e-3 * o.max_uvdiag()
+    g.schur(mu)
+    o.schur(mu)
+    assert g.factor_solve() and o.factor_solve()
+    g.backsub()
+    o.backsub()
+    assert rel(g.buffer("DP"), o.buffer("DP")) < 1e-9
+    assert rel(g.buffer("EB"), o.buffer("EB")) < 1e-11
+
+
 def test_schur_is_deterministic(P, gpu):
     sc = P.Scene(2, 7, n_pts=4000, n_cams=24)
     a = P.Context.from_scene(sc)
