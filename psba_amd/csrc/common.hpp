@@ -231,6 +231,15 @@ __device__ inline double ordered_sum(int q0, int q1, F load) {
   return acc;
 }
 
+// the same sum with fewer loads at a time where there are few (a batch of sixteen
+// clamped loads of one or two partials took most of the Schur finish)
+template <typename F>
+__device__ inline double ordered_sum_few(int q0, int q1, F load) {
+  if (q1 - q0 > 4) return ordered_sum<16>(q0, q1, load);
+  if (q1 - q0 > 1) return ordered_sum<4>(q0, q1, load);
+  return q1 > q0 ? 0.0 + load(q0) : 0.0;
+}
+
 // A problem's gate (batch: per problem through ownr; one problem: ownr may be
 // null, the gate is run[0]).
 __device__ inline bool gated_off(const unsigned char* run, const int* ownr, int i) {

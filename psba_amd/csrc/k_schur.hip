@@ -242,7 +242,7 @@ __device__ __forceinline__ void schur_finish_block(int b, const int* __restrict_
     double acc = 0.0;
     if (q >= 0) {
       const int h0 = psp[q];
-      acc = ordered_sum<16>(0, (psp[q + 1] - h0 + cpg - 1) / cpg,
+      acc = ordered_sum_few(0, (psp[q + 1] - h0 + cpg - 1) / cpg,
                             [&](int h) { return (double)part[(size_t)(h0 + h * cpg) * C2 + t]; });
     }
     double val;
@@ -257,6 +257,9 @@ __device__ __forceinline__ void schur_finish_block(int b, const int* __restrict_
     S[(size_t)(k * CNP + r) * ld + l * CNP + cc] = val;
   }
 }
+
+// threads of a finishing workgroup: one per entry of its block of S
+constexpr int finish_block(int cnp) { return cnp * cnp > 128 ? 256 : cnp * cnp > 64 ? 128 : 64; }
 
 // e_a chunks over the camera chunks: p_o = W_o z_i, column sums
 template <int CNP>
@@ -575,7 +578,7 @@ static void run_schur_t(psba_ctx* c, double mu, const R* W, R* schpart, R* eapar
                          c->cchunk_begin, c->cchunk_end, c->z, eapart, (const int2*)c->cchunk_rec);
     probe_end(c, PSBA_PROBE_SCHUR);
   }
-  const int nfin = c->n_lblocks + (c->n_pad - c->n), bs = CNP * CNP > 128 ? 256 : 128;
+  const int nfin = c->n_lblocks + (c->n_pad - c->n), bs = finish_block(CNP);
   hipLaunchKernelGGL((k_schur_ea_finish<CNP, R>), dim3(nfin + ceil_div((long)c->nc * CNP, bs)), dim3(bs), 0,
                      c->stream, c->lblock_pair, c->pair_schunk_ptr, schpart, c->U, c->fix, mu_of(c), c->n_pad,
                      c->n_lblocks, c->n, kGroups ? c->schur_group : 1, c->S, nfin, c->cam_cchunk_ptr, eapart, c->g,
@@ -660,7 +663,7 @@ __global__ __launch_bounds__(256) void k_b_schur_finish(const int* __restrict__ 
   for (int t = threadIdx.x; t < C2; t += blockDim.x) {
     const int r = t / CNP, cc = t - r * CNP;
     double acc = 0.0;
-    if (q >= 0) acc = ordered_sum<16>(psp[q], psp[q + 1], [&](int h) { return (double)part[(size_t)h * C2 + t]; });
+    if (q >= 0) acc = ordered_sum_few(psp[q], psp[q + 1], [&](int h) { return (double)part[(size_t)h * C2 + t]; });
     double val;
     if (k == l) {
       double u = U[(size_t)kg * C2 + t];
@@ -697,7 +700,7 @@ static void run_b_schur_t(psba_batch* b) {
                        dim3(256), 0, b->stream, b->items, b->schunk_b, b->schunk_e, b->obs_pt, W, b->Vinv, schpart,
                        b->schunk_prob, b->active, b->n_schunk, (const int*)nullptr, (const int4*)nullptr);
   if (b->nlb > 0)
-    hipLaunchKernelGGL((k_b_schur_finish<CNP, R>), dim3(b->nlb), dim3(CNP * CNP > 128 ? 256 : 128), 0, b->stream,
+    hipLaunchKernelGGL((k_b_schur_finish<CNP, R>), dim3(b->nlb), dim3(finish_block(CNP)), 0, b->stream,
                        b->lb_prob, b->lb_k, b->lb_l, b->lb_pair, b->psp, schpart, b->U, b->fix, b->mu, b->cam_off,
                        b->npad, b->S_off, b->active, b->S);
   hipLaunchKernelGGL(k_b_pad, dim3(b->P), dim3(256), 0, b->stream, b->cam_off, b->npad, b->S_off, CNP, b->active,
