@@ -35,7 +35,7 @@
 // plus one, so nothing is reset between launches), set by its producer behind a
 // release fence and read behind an acquire fence.  The grid is at most one
 // workgroup per CU, so that on the context's in-order stream every workgroup is
-// resident; waits are bounded (about a second, then fail bit 2).
+// resident; waits are bounded (some ten seconds, then fail bit 2).
 // d_scal[SC_FACTOR_OK] becomes 1 on success, 0 when a pivot is not positive
 // and -1 when a wait timed out.
 #include <algorithm>
