@@ -257,6 +257,13 @@ __device__ __forceinline__ void fmac_bcast(double& acc, double src, double mul) 
                    : "v"(src), "v"(mul), "n"(Q));
 }
 
+// Before the barrier behind which one wave makes the whole workgroup's stores
+// visible to other workgroups (fence, then flag): every wave waits for its own
+// stores here.  A workgroup barrier does not wait for them, and the fence of one
+// wave waits for that wave's only; a store that reached L2 after the fence's
+// write-back would be missing from what a workgroup on another XCD reads.
+__device__ __forceinline__ void drain_stores() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Workgroups of a launch go to the 8 XCDs round-robin (workgroup b to XCD
 // b % 8), each XCD with its own L2.  A grid of xcd_grid(n) workgroups with
 // item = xcd_item(b, n) gives every XCD one contiguous eighth of an n-item

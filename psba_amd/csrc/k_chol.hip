@@ -93,7 +93,8 @@ __device__ __forceinline__ void wait_flags(ull v, int* fail, ull* f0, ull* f1 = 
 
 // After the workgroup's stores: make them visible and set the flags (null: none).
 __device__ __forceinline__ void publish(ull* f0, ull v, ull* f1 = nullptr) {
-  __syncthreads();  // every wave's stores have been accepted
+  drain_stores();
+  __syncthreads();  // every wave's stores are in L2
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     if (f0) __hip_atomic_store(f0, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

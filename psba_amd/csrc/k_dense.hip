@@ -316,6 +316,7 @@ __device__ __forceinline__ double quad_xor2(double v) { return quad_perm<0x4E>(v
 // with a bounded wait (~1 s, then fail bit 2; never reached when every
 // workgroup of the launch is resident).
 __device__ __forceinline__ void grid_barrier(unsigned long long* bar, unsigned long long target, int* fail) {
+  drain_stores();
   __syncthreads();
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
