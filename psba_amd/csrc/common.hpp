@@ -264,6 +264,16 @@ __device__ __forceinline__ void fmac_bcast(double& acc, double src, double mul) 
 // write-back would be missing from what a workgroup on another XCD reads.
 __device__ __forceinline__ void drain_stores() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// Release fence towards the other workgroups, ahead of a flag: the write-back of
+// L2 has ended when it returns.  The wait is spelled out because the compiler's own
+// wait behind the write-back goes missing where it sees no access of the wave in
+// flight (after a call, say): the write-back does not count as one there, and
+// the flag could be visible before the data.
+__device__ __forceinline__ void release_stores() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  drain_stores();
+}
+
 // Workgroups of a launch go to the 8 XCDs round-robin (workgroup b to XCD
 // b % 8), each XCD with its own L2.  A grid of xcd_grid(n) workgroups with
 // item = xcd_item(b, n) gives every XCD one contiguous eighth of an n-item

@@ -96,7 +96,7 @@ __device__ __forceinline__ void publish(ull* f0, ull v, ull* f1 = nullptr) {
   drain_stores();
   __syncthreads();  // every wave's stores are in L2
   if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    release_stores();
     if (f0) __hip_atomic_store(f0, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (f1) __hip_atomic_store(f1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
         }
         if (lane == 0 && prog[kProgBad] == base + 1)
           __hip_atomic_fetch_or(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        release_stores();
         if (lane == 0) __hip_atomic_store(sy.m(k), done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       } else {
         // L_kk out
@@ -526,7 +526,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
       if (many) {
         if (w == 0) {
           xs[(size_t)k * NB + lane] = y[lane];
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+          release_stores();
           if (lane == 0) __hip_atomic_store(sy.y(), epoch + (ull)(k + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         forward(b, y, k, k + 1, 1, min(T, k + 1 + kNear));
@@ -583,7 +583,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
         const double x = b[k * NB + lane];
         if (k * NB + lane < n) dp[k * NB + lane] = x;
         xs[(size_t)k * NB + lane] = x;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        release_stores();
         if (lane == 0) __hip_atomic_store(sy.x(), epoch + (ull)(T - k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     } else if (w == 5) {

@@ -319,7 +319,7 @@ __device__ __forceinline__ void grid_barrier(unsigned long long* bar, unsigned l
   drain_stores();
   __syncthreads();
   if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    release_stores();
     const unsigned long long arrived =
         __hip_atomic_fetch_add(bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
     if (arrived < target) {
@@ -343,7 +343,7 @@ __device__ __forceinline__ void grid_barrier(unsigned long long* bar, unsigned l
 // Publish: the calling wave's earlier stores become visible first (thread 0
 // only, after the caller's __syncthreads when other waves stored).
 __device__ __forceinline__ void flag_publish(unsigned long long* f, unsigned long long v) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  release_stores();
   __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

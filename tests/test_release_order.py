@@ -56,3 +56,16 @@ def test_every_wave_drains_its_stores_before_the_barrier_of_a_release(kernels, s
             assert not STORE.match(code[k]), "stores still on their way at the barrier: %s" % code[k:barrier + 1]
             if code[k].startswith("s_waitcnt") and "vmcnt(0)" in code[k]:
                 break
+
+
+@pytest.mark.parametrize("source,least", [("k_chol.hip", 10), ("k_dense.hip", 4)])
+def test_a_release_waits_for_its_write_back(kernels, source, least):
+    """The wave's next access (the flag) only once the write-back has ended."""
+    code = kernels[source]
+    found = [k for k, line in enumerate(code) if line.startswith("buffer_wbl2")]
+    assert len(found) >= least
+    for at in found:
+        for line in code[at + 1:]:
+            assert not re.match(r"(global|flat|buffer)_", line), "no wait between write-back and %s" % line
+            if line.startswith("s_waitcnt") and "vmcnt(0)" in line:
+                break
