@@ -199,6 +199,10 @@ int psba_stage_schur(psba_ctx* ctx, double mu);
 /* Cholesky of S and the two triangular solves for dpa; *ok = 1 on success;
  * replaces SPDinv + matVec_mul, PSBA/cl_spdinv.h + PSBA/cl_linearalg.h */
 int psba_stage_factor_solve(psba_ctx* ctx, int* ok);
+/* test hook: bound of every wait between the dense solve's workgroups, in polls
+ * of a flag (multiples of 16; <= 0: the default, some ten seconds).  The first wait
+ * to reach it ends all others of the launch, and the call fails with PSBA_ERR_HIP */
+int psba_stage_wait_limit(psba_ctx* ctx, int polls);
 /* eb = gb - W^T dpa and dpb = V^-1 eb; PSBA/sba_func.cpp:1001-1117 */
 int psba_stage_backsub(psba_ctx* ctx);
 /* modified Cholesky of the current S, returns lambda = |sum E| / n;

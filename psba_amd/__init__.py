@@ -165,6 +165,7 @@ def lib():
         "psba_stage_jacobian_normal": (ct.c_int, [vp, ct.c_double, ct.c_double]),
         "psba_stage_schur": (ct.c_int, [vp, ct.c_double]),
         "psba_stage_factor_solve": (ct.c_int, [vp, ip]),
+        "psba_stage_wait_limit": (ct.c_int, [vp, ct.c_int]),
         "psba_stage_backsub": (ct.c_int, [vp]),
         "psba_stage_modchol": (ct.c_int, [vp, dp]),
         "psba_stage_refine": (ct.c_int, [vp, ct.c_double, ct.c_int]),
@@ -494,6 +495,10 @@ class Context:
         ok = ct.c_int()
         _check(lib().psba_stage_factor_solve(self._h, ct.byref(ok)), "factor_solve")
         return bool(ok.value)
+
+    def wait_limit(self, polls=0):
+        """Test hook: bound of the dense solve's waits (0: the default)."""
+        _check(lib().psba_stage_wait_limit(self._h, polls), "wait_limit")
 
     def backsub(self):
         _check(lib().psba_stage_backsub(self._h), "backsub")

@@ -274,6 +274,24 @@ __device__ __forceinline__ void release_stores() {
   drain_stores();
 }
 
+// Waits between the workgroups of a launch.  `fail` is two words: the launch's
+// status (bit 1: a pivot was not positive, bit 2: a wait timed out) and the number of
+// polls after which a wait times out.  The first wait that does ends all others
+// too, now and later in the launch (each within 16 polls), so that one bound,
+// some ten seconds by default, covers the launch.  A launch that timed out leaves
+// the status and its epoch as they are; the host clears them (dense_timed_out).
+constexpr int kWaitPolls = 1 << 24;
+// after poll number `polls` of a wait: end it unsatisfied?
+__device__ __forceinline__ bool give_up(unsigned polls, int* fail) {
+  if (polls & 15) return false;
+  const unsigned long long both =
+      __hip_atomic_load((unsigned long long*)fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (both & 2) return true;
+  if (polls < (unsigned)(both >> 32)) return false;
+  __hip_atomic_fetch_or(fail, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
 // Workgroups of a launch go to the 8 XCDs round-robin (workgroup b to XCD
 // b % 8), each XCD with its own L2.  A grid of xcd_grid(n) workgroups with
 // item = xcd_item(b, n) gives every XCD one contiguous eighth of an n-item

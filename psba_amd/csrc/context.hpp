@@ -137,7 +137,7 @@ struct psba_ctx {
   // epoch (the counter's value before the next launch)]
   double *Lf = nullptr, *yv = nullptr, *Minv = nullptr, *bw = nullptr;
   unsigned long long *sync = nullptr, *bar = nullptr;
-  int* chol_fail = nullptr;
+  int* chol_fail = nullptr;  // status of a launch and the bound of its waits (give_up)
   int chol_grid = 0;
   const double* L_cur = nullptr;  // where the last factor lives (Lf, or S after the modified Cholesky)
   double* Saux = nullptr;      // copy of S for the dogleg's recovery path (allocated on first use)
@@ -207,6 +207,7 @@ long chol_inv_len(int T);
 
 // ---- launchers (k_dense.hip) ----
 int launch_factor_solve(psba_ctx* c);                     // S -> Lf, SC_FACTOR_OK; dp[0..n) = S^-1 ea
+int dense_timed_out(psba_ctx* c);                         // (ctx.cpp) after SC_FACTOR_OK < 0: PSBA_ERR_HIP
 int launch_modchol(psba_ctx* c, double* S_src);           // SC_LAMBDA (factor in S)
 int launch_copy_S(psba_ctx* c, double* dst, const double* src);
 int launch_tri_solve(psba_ctx* c, const double* b, double* out);  // S x = b with the factor in Lf

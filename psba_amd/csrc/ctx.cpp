@@ -239,7 +239,7 @@ int psba_create(const psba_desc* d, psba_ctx** out) {
     chk(dalloc(&c->sync, (size_t)chol_sync_words(T)));
     chk(dalloc(&c->Minv, (size_t)chol_inv_len(T)));
   }
-  chk(dalloc(&c->chol_fail, (size_t)1));
+  chk(dalloc(&c->chol_fail, (size_t)2));
   c->red_part_cap = 8 * (long)std::max(ceil_div(c->no, 256), ceil_div(c->ntot, 256)) + 64;
   chk(dalloc(&c->red_part, (size_t)c->red_part_cap));
   chk(dalloc(&c->d_scal, (size_t)SC_COUNT));
@@ -255,7 +255,8 @@ int psba_create(const psba_desc* d, psba_ctx** out) {
     z(hipMemsetAsync(c->ea, 0, sizeof(double) * (size_t)c->n_pad, c->stream));
     z(hipMemsetAsync(c->dp, 0, sizeof(double) * (size_t)c->ntot, c->stream));
     z(hipMemsetAsync(c->d_scal, 0, sizeof(double) * SC_COUNT, c->stream));
-    z(hipMemsetAsync(c->chol_fail, 0, sizeof(int), c->stream));
+    static const int kStatus[2] = {0, kWaitPolls};
+    z(hipMemcpyAsync(c->chol_fail, kStatus, sizeof kStatus, hipMemcpyHostToDevice, c->stream));
     if (c->mixed()) {
       z(hipMemsetAsync(c->bar, 0, sizeof(unsigned long long) * ((size_t)3 + T), c->stream));
     } else {
@@ -486,6 +487,21 @@ int alloc_index(psba_ctx* c, long nitems, int npairs, int n_cchunk, int n_schunk
   return PSBA_OK;
 }
 
+// A dense solve whose factor status came back negative.  Nothing of that launch
+// is running any more; what it left (flags of a part of its tiles, arrivals, its
+// epoch not advanced) is cleared, so that the next launch starts as the first one did.
+int dense_timed_out(psba_ctx* c) {
+  const size_t T = (size_t)(c->n_pad / kNB);
+  PSBA_HIP_TRY(hipStreamSynchronize(c->stream));
+  if (c->mixed())
+    PSBA_HIP_TRY(hipMemsetAsync(c->bar, 0, sizeof(unsigned long long) * (3 + T), c->stream));
+  else
+    PSBA_HIP_TRY(hipMemsetAsync(c->sync, 0, sizeof(unsigned long long) * (size_t)chol_sync_words((int)T), c->stream));
+  PSBA_HIP_TRY(hipMemsetAsync(c->chol_fail, 0, sizeof(int), c->stream));
+  PSBA_HIP_TRY(hipStreamSynchronize(c->stream));
+  return fail(PSBA_ERR_HIP, "dense solve: a wait between its workgroups timed out (they were not all resident)");
+}
+
 }  // namespace psba
 
 extern "C" {
@@ -668,9 +684,17 @@ int psba_stage_factor_solve(psba_ctx* c, int* ok) {
   PSBA_TRY(launch_factor_solve(c));
   PSBA_HIP_TRY(hipMemcpyAsync(c->h_scal, c->d_scal, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, c->stream));
   PSBA_HIP_TRY(hipStreamSynchronize(c->stream));
-  if (c->h_scal[SC_FACTOR_OK] < 0.0)
-    return fail(PSBA_ERR_HIP, "dense solve: a grid-barrier wait timed out (workgroups not all resident)");
+  if (c->h_scal[SC_FACTOR_OK] < 0.0) return dense_timed_out(c);
   if (ok) *ok = c->h_scal[SC_FACTOR_OK] != 0.0;
+  return PSBA_OK;
+}
+
+int psba_stage_wait_limit(psba_ctx* c, int polls) {
+  if (!c) return fail(PSBA_ERR_ARG, "null argument");
+  PSBA_HIP_TRY(hipSetDevice(c->device));
+  const int limit = polls > 0 ? polls : kWaitPolls;
+  PSBA_HIP_TRY(hipMemcpyAsync(c->chol_fail + 1, &limit, sizeof limit, hipMemcpyHostToDevice, c->stream));
+  PSBA_HIP_TRY(hipStreamSynchronize(c->stream));
   return PSBA_OK;
 }
 

@@ -38,11 +38,7 @@ int fetch(psba_ctx* c) {
 // factorisation
 int factor_status(psba_ctx* c, bool* ok) {
   const double f = c->h_scal[SC_FACTOR_OK];
-  if (f < 0.0) {
-    set_last_error(__FILE__, __LINE__,
-                   "dense solve: a grid-barrier wait timed out (the launch's workgroups were not all resident)");
-    return PSBA_ERR_HIP;
-  }
+  if (f < 0.0) return dense_timed_out(c);
   *ok = f != 0.0;
   return PSBA_OK;
 }
@@ -205,11 +201,7 @@ int lm_device(psba_ctx* c, const psba_opts* o, int* itno, double* finalErr, psba
   PSBA_HIP_TRY(hipMemcpyAsync(c->h_lm, c->lm, sizeof(LmDev), hipMemcpyDeviceToHost, c->stream));
   PSBA_HIP_TRY(hipStreamSynchronize(c->stream));
   const LmDev st = c->h_lm[0];
-  if (st.flag < 0) {
-    set_last_error(__FILE__, __LINE__,
-                   "dense solve: a grid-barrier wait timed out (the launch's workgroups were not all resident)");
-    return st.flag;
-  }
+  if (st.flag < 0) return dense_timed_out(c);
   if (trace && len) {
     const int base = *len;
     const int take = std::max(0, std::min(st.ntrace, std::min(st.trace_cap, cap - base)));

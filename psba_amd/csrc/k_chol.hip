@@ -35,7 +35,7 @@
 // plus one, so nothing is reset between launches), set by its producer behind a
 // release fence and read behind an acquire fence.  The grid is at most one
 // workgroup per CU, so that on the context's in-order stream every workgroup is
-// resident; waits are bounded (some ten seconds, then fail bit 2).
+// resident; waits are bounded (give_up).
 // d_scal[SC_FACTOR_OK] becomes 1 on success, 0 when a pivot is not positive
 // and -1 when a wait timed out.
 #include <algorithm>
@@ -68,13 +68,9 @@ __device__ __forceinline__ ull peek(ull* f) { return __hip_atomic_load(f, __ATOM
 
 // one thread: wait until *f reaches v (bounded)
 __device__ __forceinline__ void poll(ull* f, ull v, int* fail) {
-  unsigned spins = 0;
-  while (peek(f) < v) {
+  for (unsigned polls = 1; peek(f) < v; ++polls) {
     __builtin_amdgcn_s_sleep(1);
-    if (++spins > (1u << 24)) {
-      __hip_atomic_fetch_or(fail, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      break;
-    }
+    if (give_up(polls, fail)) break;
   }
 }
 
@@ -292,7 +288,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
   const bool run = !gate || *gate;
   const int G = gridDim.x, tid = threadIdx.x, lane = tid & 63, w = wave_id(), li = lane & 15, lk = lane >> 4;
   const Sync sy{sync, T};
-  // (workgroup 1 advances it at its end, after every other workgroup's last flag)
+  // (workgroup 1 advances it at its end, after every other workgroup's last wait)
   const ull epoch = peek(sy.epoch()), done = epoch + 1;
   if (!run) return;
   auto tile = [&](double* base, int i, int j) { return base + (size_t)i * NB * ld + (size_t)j * NB; };
@@ -463,7 +459,7 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
     if (lane < n) dp[lane] = x;
     if (tid == 0) {
       const int f = __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *okp = (f & 2) ? -1.0 : (f ? 0.0 : 1.0);
+      *okp = f ? 0.0 : 1.0;  // (there is nothing to wait for)
       __hip_atomic_store(fail, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     return;
@@ -600,8 +596,10 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
     if (tid == 0) {
       const int f = __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       *okp = (f & 2) ? -1.0 : (f ? 0.0 : 1.0);
-      __hip_atomic_store(fail, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(sy.epoch(), epoch + (ull)(T + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!(f & 2)) {
+        __hip_atomic_store(fail, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(sy.epoch(), epoch + (ull)(T + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
     return;
   }

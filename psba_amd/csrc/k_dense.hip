@@ -313,8 +313,8 @@ __device__ __forceinline__ double quad_xor2(double v) { return quad_perm<0x4E>(v
 // waits until the counter reaches `target`.  The add returns the count, so the
 // workgroup that arrives last (workgroup 0, which carries the diagonal chain)
 // sees at once that the others are in and does not poll; the others poll
-// with a bounded wait (~1 s, then fail bit 2; never reached when every
-// workgroup of the launch is resident).
+// with a bounded wait (give_up; the bound is never reached when every workgroup
+// of the launch is resident).
 __device__ __forceinline__ void grid_barrier(unsigned long long* bar, unsigned long long target, int* fail) {
   drain_stores();
   __syncthreads();
@@ -323,13 +323,9 @@ __device__ __forceinline__ void grid_barrier(unsigned long long* bar, unsigned l
     const unsigned long long arrived =
         __hip_atomic_fetch_add(bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
     if (arrived < target) {
-      unsigned spins = 0;
-      while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+      for (unsigned polls = 1; __hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target; ++polls) {
         __builtin_amdgcn_s_sleep(2);
-        if (++spins > (1u << 24)) {
-          __hip_atomic_fetch_or(fail, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          break;
-        }
+        if (give_up(polls, fail)) break;
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -355,13 +351,9 @@ __device__ __forceinline__ void flag_wait(unsigned long long* f, unsigned long l
                                           unsigned long long seen = 0) {
   if (threadIdx.x == 0) {
     if (seen < v) {
-      unsigned spins = 0;
-      while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) {
+      for (unsigned polls = 1; __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v; ++polls) {
         __builtin_amdgcn_s_sleep(2);
-        if (++spins > (1u << 24)) {
-          __hip_atomic_fetch_or(fail, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          break;
-        }
+        if (give_up(polls, fail)) break;
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -1294,9 +1286,11 @@ __global__ __launch_bounds__(256) void k_chol_phases(double* __restrict__ A, int
     // cleared for the next launch (every other workgroup is past its last
     // wait: workgroup 0 consumed every helper's last flag), and the epoch of
     // the next launch: this launch's T barriers of G arrivals each
-    __hip_atomic_store(fail, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(bar + 2 + T, bar_base + (unsigned long long)G * T, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    if (!(f & 2)) {
+      __hip_atomic_store(fail, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(bar + 2 + T, bar_base + (unsigned long long)G * T, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 }
 

@@ -6,6 +6,8 @@ reduced right-hand side, factor/solve, back-substitution) and whole drivers
 every camera model (cnp 6, 9, 11, 16).  The plain FP64 path must reproduce
 the oracle's per-trial cost and final parameters within 1e-9 relative.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -324,6 +326,56 @@ def test_dense_factor_at_tile_edges(P, gpu, cnp, n_cams):
     x, L = runs[0]
     assert rel(x, np.linalg.solve(S, b)) < 1e-9
     assert rel(L, np.linalg.cholesky(S)) < 1e-11
+
+
+# a workgroup per tile, and several tiles each; the bound is shorter than any of these launches
+@pytest.mark.parametrize("cnp,n_cams,prec", [(16, 64, "fp64"), (9, 300, "fp64"), (16, 64, "mixed"), (9, 300, "mixed")])
+def test_dense_solve_after_a_timed_out_wait(P, gpu, cnp, n_cams, prec):
+    """The first wait to run out ends the launch and the call with an error, and
+    the next launch is as good as the first one of a new context."""
+    rng = np.random.default_rng(n_cams)
+    n = cnp * n_cams
+    S, b = spd(n, rng), rng.standard_normal(n)
+    with P.Context(cnp, n_cams, 4, 8, precision=P.PREC_MIXED if prec == "mixed" else P.PREC_FP64) as c:
+        c.load_S(S, b)
+        ok, first = c.factor_only()
+        assert ok
+        for _ in range(2):
+            c.wait_limit(16)
+            c.load_S(S, b)
+            start = time.perf_counter()
+            with pytest.raises(P.PsbaError, match="timed out"):
+                c.factor_only()
+            # 16 polls (some 10 us) a wait, at most four waits a tile column
+            assert time.perf_counter() - start < 1.0
+            c.wait_limit()
+            for _ in range(3):
+                c.load_S(S, b)
+                ok, x = c.factor_only()
+                assert ok and np.array_equal(x, first)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_solve_after_a_timed_out_wait(P, gpu, prec):
+    """The same through the LM drivers, which decide on the device or on the host."""
+    sc = P.Scene(2, 5, n_cams=120, n_pts=2000, outlier_frac=0.0)
+    kw = dict(max_iter=4, flags=P.FLAG_NO_HANDOFF)
+    with P.Context.from_scene(sc, precision=P.PREC_MIXED if prec == "mixed" else P.PREC_FP64) as c:
+        c.snapshot()
+        c.levmar(**kw)
+        want = c.read_params()
+        for flags in (P.FLAG_NO_HANDOFF, P.FLAG_NO_HANDOFF | P.FLAG_HOST_CONTROL):
+            c.restore()
+            c.itno = 0
+            c.wait_limit(16)
+            with pytest.raises(P.PsbaError, match="timed out"):
+                c.levmar(max_iter=4, flags=flags)
+            c.wait_limit()
+            c.restore()
+            c.itno = 0
+            c.levmar(max_iter=4, flags=flags)
+            got = c.read_params()
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("n_cams", [7, 40])
