@@ -35,7 +35,11 @@
 // plus one, so nothing is reset between launches), set by its producer behind a
 // release fence and read behind an acquire fence.  The grid is at most one
 // workgroup per CU, so that on the context's in-order stream every workgroup is
-// resident; waits are bounded (give_up).
+// resident.  Beside another stream's launches they may not all be: up to T = 22 a
+// tile waits only for lower-numbered workgroups, and all but the last T - 4 owners
+// leave when their tile is done, so that the others find room (two contexts of 16
+// tiles together have 272 workgroups); from T = 23 on a launch needs the
+// whole device, and one that does not get it ends after the bounded waits (give_up).
 // d_scal[SC_FACTOR_OK] becomes 1 on success, 0 when a pivot is not positive
 // and -1 when a wait timed out.
 #include <algorithm>
@@ -862,8 +866,9 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
   }
   // ---- helpers of the back substitution: row i's terms x_j, j = T - 1 .. i + kNear + 1
   // (x_{T-1} is published after every L_ik, so the tiles can be loaded ahead of the
-  // x that they wait for)
-  for (int i = o; i + kNear + 1 < T; i += G - 2) {
+  // x that they wait for).  With a workgroup per tile the last owners do it, and
+  // the others leave with their tile.
+  for (int i = many ? o : G - 3 - o; i + kNear + 1 < T; i += G - 2) {
     double s = 0.0;
     TileRegs<4> l;
     for (int j = T - 1; j >= i + kNear + 1; --j) {

@@ -6,7 +6,9 @@ reduced right-hand side, factor/solve, back-substitution) and whole drivers
 every camera model (cnp 6, 9, 11, 16).  The plain FP64 path must reproduce
 the oracle's per-trial cost and final parameters within 1e-9 relative.
 """
+import threading
 import time
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -326,6 +328,37 @@ def test_dense_factor_at_tile_edges(P, gpu, cnp, n_cams):
     x, L = runs[0]
     assert rel(x, np.linalg.solve(S, b)) < 1e-9
     assert rel(L, np.linalg.cholesky(S)) < 1e-11
+
+
+# together more workgroups than compute units (256): 2 x 136, 4 x 66
+@pytest.mark.parametrize("cnp,n_cams,contexts", [(16, 64, 2), (16, 44, 4)])
+def test_dense_solves_side_by_side(P, gpu, cnp, n_cams, contexts):
+    rng = np.random.default_rng(n_cams)
+    n = cnp * n_cams
+    S, b = spd(n, rng), rng.standard_normal(n)
+    ctxs = [P.Context(cnp, n_cams, 4, 8) for _ in range(contexts)]
+    try:
+        for c in ctxs:
+            c.wait_limit(1 << 20)  # (about a second)
+        ctxs[0].load_S(S, b)
+        ok, want = ctxs[0].factor_only()
+        assert ok
+        start = threading.Barrier(contexts)
+
+        def work(c):
+            out = []
+            for _ in range(25):
+                c.load_S(S, b)
+                start.wait(30)
+                out.append(c.factor_only())
+            return out
+
+        with ThreadPoolExecutor(contexts) as ex:
+            for out in ex.map(work, ctxs):
+                assert all(ok and np.array_equal(x, want) for ok, x in out)
+    finally:
+        for c in ctxs:
+            c.close()
 
 
 # a workgroup per tile, and several tiles each; the bound is shorter than any of these launches
