@@ -589,6 +589,11 @@ int psba_batch_commit(psba_batch* b) {
   size_t in_bytes = 0;
   psba_batch hv;  // views into the staging image
   const size_t need = carve(&hv, z, C, R, nullptr, &in_bytes);
+  // from here on the last solve's buffers go; should the commit fail, neither a
+  // result nor a launch may use what is left of them
+  b->committed = false;
+  b->finished = false;
+  drop_read_ahead(b);
   PSBA_TRY(free_graph(b));
   PSBA_HIP_TRY(hipEventSynchronize(b->ev_staged));  // the previous upload has left the staging image
   if (need > b->arena_bytes) {
@@ -598,6 +603,7 @@ int psba_batch_commit(psba_batch* b) {
     b->arena_bytes = 0;
     hipError_t e = hipMalloc((void**)&b->arena, need);
     if (e != hipSuccess) {
+      (void)hipGetLastError();  // (or the next launch check would report it)
       b->arena = nullptr;
       return bfail(PSBA_ERR_NOMEM, "hipMalloc of %zu bytes failed: %s", need, hipGetErrorString(e));
     }
@@ -609,6 +615,7 @@ int psba_batch_commit(psba_batch* b) {
     b->staging_bytes = 0;
     hipError_t e = hipHostMalloc((void**)&b->staging, in_bytes, hipHostMallocDefault);
     if (e != hipSuccess) {
+      (void)hipGetLastError();
       b->staging = nullptr;
       return bfail(PSBA_ERR_NOMEM, "pinned allocation of %zu bytes failed: %s", in_bytes, hipGetErrorString(e));
     }
@@ -621,6 +628,7 @@ int psba_batch_commit(psba_batch* b) {
     b->h_stat_cap = 0;
     hipError_t e = hipHostMalloc((void**)&b->h_stat, sizeof(BatchStat) * 2 * (size_t)(P + 1), hipHostMallocDefault);
     if (e != hipSuccess) {
+      (void)hipGetLastError();
       b->h_stat = nullptr;
       return bfail(PSBA_ERR_NOMEM, "pinned allocation failed: %s", hipGetErrorString(e));
     }
@@ -751,8 +759,6 @@ int psba_batch_commit(psba_batch* b) {
   PSBA_HIP_TRY(hipMemsetAsync(b->Lf, 0, sizeof(double) * (size_t)z.S_len, b->stream));
   PSBA_HIP_TRY(hipMemsetAsync(b->dp, 0, sizeof(double) * (size_t)(z.N + 3 * z.NP), b->stream));
   b->committed = true;
-  b->finished = false;
-  drop_read_ahead(b);
   return PSBA_OK;
 }
 

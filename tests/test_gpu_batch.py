@@ -286,3 +286,52 @@ def test_results_in_order_equal_results_out_of_order(P, gpu, n_pts):
             assert any(not np.array_equal(u["pts"], f["pts"]) for u, f in zip(up, first))
         first = up
     b.close()
+
+
+def test_after_a_commit_that_fails(P, gpu):
+    """More device memory than there is: neither the earlier solve's results nor
+    a launch may use its freed buffers, and the batch can be filled again."""
+    scenes = [window(P, k, n_cams=5, n_pts=n) for k, n in enumerate((40, 7, 300))]
+    cams = 8190 // 6  # a problem's dense blocks: 2 x 8192 x 8192 doubles, 1.07 GB
+    iidx, jidx = np.repeat(np.arange(2), 3), np.tile(np.arange(3), 2)
+    with P.Batch(6) as b:
+        for sc in scenes:
+            b.add_scene(sc)
+        b.commit()
+        b.solve(**OPTS)
+        first = [b.result(s) for s in range(len(scenes))]
+        for _ in range(300):
+            b.add(np.ones(5 * cams), np.zeros(12), np.tile([1.0, 0, 0, 0], cams), np.zeros(6 * cams), np.ones(6), iidx,
+                  jidx)
+        with pytest.raises(P.PsbaError, match="memory"):
+            b.commit()
+        for call in (lambda: b.result(0), lambda: b.launch(), lambda: b.poll(), lambda: b.elapsed()):
+            with pytest.raises(P.PsbaError):
+                call()
+        b.reset()
+        for sc in scenes:
+            b.add_scene(sc)
+        b.commit()
+        b.solve(**OPTS)
+        for s, f in enumerate(first):
+            same(b.result(s), f)
+
+
+def test_results_stay_until_a_commit_replaces_them(P, gpu):
+    """A problem added after a solve leaves its results; a commit ends them."""
+    scenes = [window(P, k, n_cams=5, n_pts=n) for k, n in enumerate((40, 7, 300))]
+    with P.Batch(6) as b:
+        for sc in scenes:
+            b.add_scene(sc)
+        b.commit()
+        b.solve(**OPTS)
+        first = [b.result(s) for s in range(3)]
+        b.add_scene(window(P, 3, n_cams=6, n_pts=90))
+        for s in (0, 2, 1):
+            same(b.result(s), first[s])
+        b.commit()
+        with pytest.raises(P.PsbaError):
+            b.result(0)
+        b.solve(**OPTS)
+        for s in range(3):
+            same(b.result(s), first[s])
