@@ -77,7 +77,9 @@ int psba_batch_poll(psba_batch* b);
 int psba_batch_solve(psba_batch* b, const psba_opts* o, int* rounds);
 
 /* Per-problem outcome: the ITER_* code, iterations, initial and final sum of
- * squared residuals, and (if non-NULL) the final parameters. */
+ * squared residuals, and (if non-NULL) the final parameters.  Several threads
+ * may read results of a finished solve at once; every other call needs the
+ * batch to itself. */
 int psba_batch_result(psba_batch* b, int slot, int* code, int* itno, double* init_err, double* final_err,
                       double* cams, double* pts);
 

@@ -297,11 +297,38 @@ int launch_round(psba_batch* b) {
 // what was read ahead is no longer what the device holds
 void drop_read_ahead(psba_batch* b) {
   std::lock_guard<std::mutex> lock(b->ahead_mtx);
-  b->ahead_lo = b->ahead_hi = 0;
-  b->last_slot = -1;
+  b->ahead_cams = b->ahead_pts = psba_batch::ReadAhead();
 }
 
 constexpr size_t kReadAhead = (size_t)4 << 20;  // bytes of results fetched together
+
+// Slot `slot` of cams or pts (`dev`, `stride` values for each of off[slot] ..
+// off[slot + 1] - 1) into the caller's memory.  Asked for after the slot before it, it
+// brings the next ones along, up to kReadAhead bytes, into their places in `image`: a
+// copy a slot into pageable memory took 20 us (512 windows, cameras and points: 20 of
+// 48 ms).  A slot on its own is copied straight to the caller.
+int read_slot(psba_batch* b, psba_batch::ReadAhead& a, const double* dev, double* image, size_t stride,
+              const std::vector<int>& off, int slot, double* out) {
+  const size_t at = stride * off[slot], n = stride * off[slot + 1] - at;
+  const bool next = slot > 0 && slot == a.last + 1;
+  a.last = slot;
+  if (slot < a.lo || slot >= a.hi) {
+    int hi = slot + 1;
+    auto bytes = [&](int h) { return sizeof(double) * (stride * off[h] - at); };
+    while (next && hi < b->P && bytes(hi + 1) <= kReadAhead) ++hi;
+    if (hi == slot + 1) {
+      PSBA_HIP_TRY(hipMemcpy(out, dev + at, sizeof(double) * n, hipMemcpyDeviceToHost));
+      return PSBA_OK;
+    }
+    a.lo = a.hi = 0;
+    PSBA_HIP_TRY(hipMemcpyAsync(image + at, dev + at, bytes(hi), hipMemcpyDeviceToHost, b->stream));
+    PSBA_HIP_TRY(hipStreamSynchronize(b->stream));
+    a.lo = slot;
+    a.hi = hi;
+  }
+  std::copy(image + at, image + at + n, out);
+  return PSBA_OK;
+}
 
 // wait for the rounds queued behind the last check and read the solve's time
 int settle(psba_batch* b) {
@@ -818,45 +845,15 @@ int psba_batch_result(psba_batch* b, int slot, int* code, int* itno, double* ini
   if (!b->finished) return bfail(PSBA_ERR_STATE, "no finished solve");
   if (slot < 0 || slot >= b->P) return bfail(PSBA_ERR_ARG, "slot %d out of range", slot);
   PSBA_HIP_TRY(hipSetDevice(b->device));
+  std::lock_guard<std::mutex> lock(b->ahead_mtx);
   PSBA_TRY(settle(b));
   const BatchStat& st = batch_final_stat(b)[slot + 1];
   if (code) *code = st.code;
   if (itno) *itno = st.itno;
   if (init_err) *init_err = st.init_err;
   if (final_err) *final_err = st.cost;
-  if (!cams && !pts) return PSBA_OK;
-  const size_t C = (size_t)b->cnp, N = (size_t)b->N;
-  const size_t c0 = C * b->h_cam_off[slot], c1 = C * b->h_cam_off[slot + 1];
-  const size_t p0 = 3 * (size_t)b->h_pt_off[slot], p1 = 3 * (size_t)b->h_pt_off[slot + 1];
-  std::lock_guard<std::mutex> lock(b->ahead_mtx);
-  double* const image = (double*)b->staging;
-  if (slot < b->ahead_lo || slot >= b->ahead_hi) {
-    if (slot != b->last_slot + 1 || slot == 0) {
-      b->last_slot = slot;
-      if (cams) PSBA_HIP_TRY(hipMemcpy(cams, b->cams + c0, sizeof(double) * (c1 - c0), hipMemcpyDeviceToHost));
-      if (pts) PSBA_HIP_TRY(hipMemcpy(pts, b->pts + p0, sizeof(double) * (p1 - p0), hipMemcpyDeviceToHost));
-      return PSBA_OK;
-    }
-    // one slot after another: this one and the next, up to kReadAhead bytes.  Two
-    // copies a slot into pageable memory took 40 us a slot (512 windows: 20 of 48 ms).
-    int hi = slot + 1;
-    auto bytes = [&](int h) {
-      return sizeof(double) * (C * (size_t)(b->h_cam_off[h] - b->h_cam_off[slot]) +
-                               3 * (size_t)(b->h_pt_off[h] - b->h_pt_off[slot]));
-    };
-    while (hi < b->P && bytes(hi + 1) <= kReadAhead) ++hi;
-    b->ahead_lo = b->ahead_hi = 0;
-    const size_t c2 = C * b->h_cam_off[hi], p2 = 3 * (size_t)b->h_pt_off[hi];
-    PSBA_HIP_TRY(hipMemcpyAsync(image + c0, b->cams + c0, sizeof(double) * (c2 - c0), hipMemcpyDeviceToHost, b->stream));
-    PSBA_HIP_TRY(
-        hipMemcpyAsync(image + N + p0, b->pts + p0, sizeof(double) * (p2 - p0), hipMemcpyDeviceToHost, b->stream));
-    PSBA_HIP_TRY(hipStreamSynchronize(b->stream));
-    b->ahead_lo = slot;
-    b->ahead_hi = hi;
-  }
-  b->last_slot = slot;
-  if (cams) std::copy(image + c0, image + c1, cams);
-  if (pts) std::copy(image + N + p0, image + N + p1, pts);
+  if (cams) PSBA_TRY(read_slot(b, b->ahead_cams, b->cams, (double*)b->staging, (size_t)b->cnp, b->h_cam_off, slot, cams));
+  if (pts) PSBA_TRY(read_slot(b, b->ahead_pts, b->pts, (double*)b->staging + b->N, 3, b->h_pt_off, slot, pts));
   return PSBA_OK;
 }
 

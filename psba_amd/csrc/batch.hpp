@@ -63,11 +63,15 @@ struct psba_batch {
   char* staging = nullptr;
   size_t staging_bytes = 0;
   hipEvent_t ev_staged = nullptr;
-  // results read ahead (psba_batch_result): the parameters of slots [ahead_lo,
-  // ahead_hi) of the finished solve, in the staging image at the places that cams
-  // and pts have from its start; last_slot: the one asked for last
+  // results read ahead (psba_batch_result), cameras and points each as they are
+  // asked for: slots [lo, hi) of the finished solve, in the staging image at the
+  // places that cams, and pts behind them, have from its start; last: the slot asked
+  // for last
+  struct ReadAhead {
+    int lo = 0, hi = 0, last = -1;
+  };
   std::mutex ahead_mtx;
-  int ahead_lo = 0, ahead_hi = 0, last_slot = -1;
+  ReadAhead ahead_cams, ahead_pts;
 
   // problem data
   double *K = nullptr, *q0 = nullptr, *meas = nullptr, *cams = nullptr, *pts = nullptr;

@@ -14,6 +14,9 @@
 * The mixed-precision batch reaches the FP64 batch's final cost within 1e-6
   relative.
 """
+import ctypes as ct
+import time
+
 import numpy as np
 import pytest
 
@@ -335,3 +338,55 @@ def test_results_stay_until_a_commit_replaces_them(P, gpu):
         b.solve(**OPTS)
         for s in range(3):
             same(b.result(s), first[s])
+
+
+def read_one(P, b, slot, cams, pts):
+    """psba_batch_result with either array left out (null)."""
+    code, it, ie, fe = ct.c_int(), ct.c_int(), ct.c_double(), ct.c_double()
+    ptr = [None if a is None else a.ctypes.data_as(ct.POINTER(ct.c_double)) for a in (cams, pts)]
+    assert P.lib().psba_batch_result(b._h, slot, ct.byref(code), ct.byref(it), ct.byref(ie), ct.byref(fe), *ptr) == 0
+
+
+def test_results_of_cameras_or_points_alone(P, gpu):
+    """Either array in any order, alone, in turn or with the other."""
+    sizes = [(5, 40), (6, 7), (30, 4000)] + [(5, 50000)] * 5 + [(9, 180000), (5, 200)]
+    scenes = [window(P, k, n_cams=c, n_pts=n) for k, (c, n) in enumerate(sizes)]
+    with P.Batch(6) as b:
+        for sc in scenes:
+            b.add_scene(sc)
+        b.commit()
+        b.solve(max_iter=2)
+        want = [b.result(s) for s in reversed(range(len(sizes)))][::-1]
+        up = list(range(len(sizes)))
+        for order, cams, pts in [(up, 1, 0), (up, 0, 1), (up[::-1], 1, 0), (up, 1, 1), (up[3:], 0, 1), (up, "even", "odd"),
+                                 (up, 1, "odd")]:
+            for s in order:
+                take = [x == 1 or x == ("even", "odd")[s % 2] for x in (cams, pts)]
+                c = np.full_like(want[s]["cams"], np.nan) if take[0] else None
+                p = np.full_like(want[s]["pts"], np.nan) if take[1] else None
+                read_one(P, b, s, c, p)
+                assert c is None or np.array_equal(c, want[s]["cams"])
+                assert p is None or np.array_equal(p, want[s]["pts"])
+
+
+def test_cameras_alone_do_not_wait_for_points(P, gpu):
+    """Cameras of slots with many points, in ascending order: as cheap as one by
+    one (a few hundred bytes each), not a copy of their points (3.8 MB each)."""
+    with P.Batch(6) as b:
+        for k in range(8):
+            b.add_scene(window(P, k, n_cams=5, n_pts=160000))
+        b.commit()
+        b.solve(max_iter=1)
+        cams = np.empty(30)
+
+        def seconds(order):
+            best = 1.0
+            for _ in range(20):
+                start = time.perf_counter()
+                for s in order:
+                    read_one(P, b, s, cams, None)
+                best = min(best, time.perf_counter() - start)
+            return best
+
+        one_by_one = seconds(range(7, -1, -1))
+        assert seconds(range(8)) < 1.5 * one_by_one
