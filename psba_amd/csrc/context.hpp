@@ -106,7 +106,7 @@ struct psba_ctx {
   // workgroup index gives (built by build_schur_slots)
   int2* cchunk_rec = nullptr;
   int* pt_order = nullptr;      // points by descending track length (ties: ascending id)
-  int n_long = 0;               // of them with kLongTrack observations or more
+  int n_long = 0;               // points with kLongTrack observations or more
   double sum_t2 = 0;            // sum over points of track length squared
   double entry_cost = 0;        // SSE at the entry of the last psba_levmar call
 
@@ -196,7 +196,7 @@ int launch_axpby(psba_ctx* c, double* out, double alpha, const double* a, double
 
 // ---- launchers (k_schur.hip) ----
 int launch_schur(psba_ctx* c, double mu);                 // S (lower), ea
-int build_point_order(psba_ctx* c);                        // pt_order, n_long (index builds)
+int build_point_order(psba_ctx* c);                        // pt_order (index builds)
 int build_schur_slots(psba_ctx* c);                        // item_rec and sgroup or slot_items, cchunk_rec (index builds)
 int launch_ea_rhs(psba_ctx* c, const double* ga, const double* z, double* out);  // ga - sum W z
 

@@ -87,13 +87,15 @@ __global__ void k_chunk_counts(const int* __restrict__ ptr, int n, int CH, int* 
   if (j < n) cnt[j] = (ptr[j + 1] - ptr[j] + CH - 1) / CH;
 }
 
+// items of each point; sums: of t squared, and the number of long tracks
 __global__ void k_item_counts(const int* __restrict__ pt_ptr, int np, long long* __restrict__ cnt,
-                              long long* __restrict__ t2) {
+                              unsigned long long* __restrict__ sums) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const long long t = pt_ptr[i + 1] - pt_ptr[i];
   cnt[i] = t * (t + 1) / 2;
-  if (t) atomicAdd((unsigned long long*)t2, (unsigned long long)(t * t));
+  if (t) atomicAdd(sums, (unsigned long long)(t * t));
+  if (t >= kLongTrack) atomicAdd(sums + 1, 1ull);
 }
 
 // launch key of each pair chunk (its first item's cameras and point)
@@ -256,21 +258,23 @@ int psba_set_index_device(psba_ctx* c, const int* iidx, const int* jidx) {
   IX_TRY(rocprim::exclusive_scan(nullptr, tb, ccnt.p, ccp.p, 0, (size_t)nc, rocprim::plus<int>(), st));
   PSBA_TRY(tmp.ensure(tb));
   IX_TRY(rocprim::exclusive_scan(tmp.p, tb, ccnt.p, ccp.p, 0, (size_t)nc, rocprim::plus<int>(), st));
-  // items per point and their offsets; sum of t^2
-  DevBuf<long long> icnt, ioff, t2;
+  // items per point and their offsets; sum of t^2, long tracks
+  DevBuf<long long> icnt, ioff;
+  DevBuf<unsigned long long> sums;
   PSBA_TRY(icnt.alloc(np));
   PSBA_TRY(ioff.alloc(np));
-  PSBA_TRY(t2.alloc(2));
-  IX_TRY(hipMemsetAsync(t2.p, 0, sizeof(long long) * 2, st));
-  hipLaunchKernelGGL(k_item_counts, grid(np), dim3(256), 0, st, ptptr.p, np, icnt.p, t2.p);
+  PSBA_TRY(sums.alloc(2));
+  IX_TRY(hipMemsetAsync(sums.p, 0, sizeof(unsigned long long) * 2, st));
+  hipLaunchKernelGGL(k_item_counts, grid(np), dim3(256), 0, st, ptptr.p, np, icnt.p, sums.p);
   IX_TRY(rocprim::exclusive_scan(nullptr, tb, icnt.p, ioff.p, 0LL, (size_t)np, rocprim::plus<long long>(), st));
   PSBA_TRY(tmp.ensure(tb));
   IX_TRY(rocprim::exclusive_scan(tmp.p, tb, icnt.p, ioff.p, 0LL, (size_t)np, rocprim::plus<long long>(), st));
-  long long h_last[2] = {0, 0}, h_t2 = 0;
+  long long h_last[2] = {0, 0};
+  unsigned long long h_sums[2] = {0, 0};
   int h_cc[2] = {0, 0};
   IX_TRY(hipMemcpyAsync(&h_last[0], ioff.p + (np - 1), sizeof(long long), hipMemcpyDeviceToHost, st));
   IX_TRY(hipMemcpyAsync(&h_last[1], icnt.p + (np - 1), sizeof(long long), hipMemcpyDeviceToHost, st));
-  IX_TRY(hipMemcpyAsync(&h_t2, t2.p, sizeof(long long), hipMemcpyDeviceToHost, st));
+  IX_TRY(hipMemcpyAsync(h_sums, sums.p, sizeof h_sums, hipMemcpyDeviceToHost, st));
   IX_TRY(hipMemcpyAsync(&h_cc[0], ccp.p + (nc - 1), sizeof(int), hipMemcpyDeviceToHost, st));
   IX_TRY(hipMemcpyAsync(&h_cc[1], ccnt.p + (nc - 1), sizeof(int), hipMemcpyDeviceToHost, st));
   IX_TRY(hipStreamSynchronize(st));
@@ -330,7 +334,8 @@ int psba_set_index_device(psba_ctx* c, const int* iidx, const int* jidx) {
 
   // the context's buffers
   PSBA_TRY(alloc_index(c, (long)nitems, npairs, n_cchunk, n_schunk));
-  c->sum_t2 = (double)h_t2;
+  c->sum_t2 = (double)h_sums[0];
+  c->n_long = (int)h_sums[1];
   IX_TRY(hipMemcpyAsync(c->obs_pt, d_i.p, sizeof(int) * no, hipMemcpyDeviceToDevice, st));
   IX_TRY(hipMemcpyAsync(c->obs_cam, d_j.p, sizeof(int) * no, hipMemcpyDeviceToDevice, st));
   IX_TRY(hipMemcpyAsync(c->pt_ptr, ptptr.p, sizeof(int) * (np + 1), hipMemcpyDeviceToDevice, st));
@@ -497,18 +502,6 @@ int build_schur_slots(psba_ctx* c) {
 // Points by descending track length, ties in ascending id (a stable radix
 // sort).  The back substitution takes its points in this order, so that the
 // points one wave handles in lockstep have tracks of similar length.
-// how many of the points, in that order, have tracks of at least kLongTrack
-__global__ void k_long_tracks(const int* __restrict__ order, const int* __restrict__ pt_ptr, int np,
-                              int* __restrict__ n) {
-  int lo = 0, hi = np;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1, i = order[mid];
-    if (pt_ptr[i + 1] - pt_ptr[i] >= kLongTrack) lo = mid + 1;
-    else hi = mid;
-  }
-  *n = lo;
-}
-
 int build_point_order(psba_ctx* c) {
   const int np = c->np;
   hipStream_t st = c->stream;
@@ -523,9 +516,7 @@ int build_point_order(psba_ctx* c) {
   Scratch tmp;
   PSBA_TRY(tmp.ensure(tb));
   IX_TRY(rocprim::radix_sort_pairs(tmp.p, tb, key.p, key_s.p, val.p, c->pt_order, (size_t)np, 0, 32, st));
-  hipLaunchKernelGGL(k_long_tracks, dim3(1), dim3(1), 0, st, c->pt_order, c->pt_ptr, np, val.p);
   IX_TRY(hipGetLastError());
-  IX_TRY(hipMemcpyAsync(&c->n_long, val.p, sizeof(int), hipMemcpyDeviceToHost, st));
   IX_TRY(hipStreamSynchronize(st));  // the temporaries are freed on return
   return PSBA_OK;
 }

@@ -112,3 +112,20 @@ def test_generate_idxs_device_scene(P, gpu):
     for x, y in zip(h[:4], d):
         assert np.array_equal(x, y)
     assert np.array_equal(d[0], sc.iidx) and np.array_equal(d[1], sc.jidx)
+
+
+# tracks on both sides of seven observations, from which on several lanes share a point
+@pytest.mark.parametrize("config,kw", [(1, dict(n_cams=9, n_pts=30)), (2, dict(n_cams=6, n_pts=200)),
+                                       (2, dict(n_cams=60, n_pts=700))])
+def test_steps_of_long_tracks_are_the_same_with_either_index(P, gpu, config, kw):
+    sc = P.Scene(config, 12, **kw)
+    out = []
+    for c in build_pair(P, sc, sc.iidx, sc.jidx):
+        c.upload(sc.K, sc.meas, sc.q0, sc.cams, sc.pts)
+        c.set_fixed(sc.fixmask)
+        c.jacobian_normal(1.0, 1.0)
+        c.schur(1e3)
+        assert c.factor_solve()
+        c.backsub()
+        out.append((c.buffer("DP"), c.buffer("EB")))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
