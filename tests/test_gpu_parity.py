@@ -330,6 +330,69 @@ def test_dense_factor_at_tile_edges(P, gpu, cnp, n_cams):
     assert rel(L, np.linalg.cholesky(S)) < 1e-11
 
 
+def ill_conditioned(kind, n, cond, rng):
+    if kind == "spectrum":
+        A = spd(n, rng, cond)
+    elif kind == "tiles":  # every 64 x 64 diagonal tile
+        A, d = spd(n, rng, 1e2), np.logspace(0, -np.log10(cond) / 2, 64)[np.arange(n) % 64]
+        A = A * d * d[:, None]
+    elif kind == "columns":  # badly scaled
+        A, d = spd(n, rng, 1e4), np.sqrt(cond) ** rng.uniform(-0.5, 0.5, n)
+        A = A * d * d[:, None]
+    else:  # seven directions that are nearly free
+        Q, _ = np.linalg.qr(rng.standard_normal((n, 7)))
+        A = spd(n, rng, 1e3)
+        A = A - Q @ (Q.T @ A)
+        A = A - (A @ Q) @ Q.T + Q @ Q.T / cond
+    return np.tril(A) + np.tril(A, -1).T
+
+
+def check_factor_and_solution(S, b, x, L, rows):
+    """Backward errors within the textbook bounds of Cholesky by substitution:
+    |L L^T - S| <= (n + 1) eps |L| |L^T| (in the given rows), |S x - b| <= (3 n + 1) eps |S| |x|."""
+    n, eps = b.size, np.finfo(np.float64).eps
+    assert np.all(np.abs(L[rows] @ L.T - S[rows]) <= (n + 1) * eps * (np.abs(L[rows]) @ np.abs(L).T))
+    r = (S.astype(np.longdouble) @ x.astype(np.longdouble) - b).astype(np.float64)
+    assert np.max(np.abs(r)) <= (3 * n + 1) * eps * np.max(np.abs(S).sum(1)) * np.max(np.abs(x))
+
+
+# the tiles' inverses stand in for substitutions: no worse where the tiles, or the
+# whole system, are nearly singular
+@pytest.mark.parametrize("cnp,n_cams", [(6, 10), (9, 36), (9, 88), (16, 88)])
+@pytest.mark.parametrize("kind,cond", [("spectrum", 1e10), ("spectrum", 1e12), ("spectrum", 1e14), ("tiles", 1e12),
+                                       ("tiles", 1e20), ("columns", 1e20), ("directions", 1e12)])
+def test_dense_solve_of_ill_conditioned_systems(P, gpu, cnp, n_cams, kind, cond):
+    n = cnp * n_cams
+    rng = np.random.default_rng(n)
+    S, b = ill_conditioned(kind, n, cond, rng), rng.standard_normal(n)
+    with P.Context(cnp, n_cams, 4, 8) as c:
+        c.load_S(S, b)
+        ok, x = c.factor_only()
+        assert ok
+        check_factor_and_solution(S, b, x, np.tril(c.buffer("L").reshape(n, n)), np.arange(n))
+
+
+# 67 and 128 tiles a side, the largest order: ten and more than thirty tiles an owner
+@pytest.mark.parametrize("cnp,n_cams", [(16, 268), (16, 512)])
+def test_dense_solve_of_large_systems(P, gpu, cnp, n_cams):
+    n = cnp * n_cams
+    rng = np.random.default_rng(n)
+    S = np.tril(rng.standard_normal((n, n)) * (0.5 / np.sqrt(n)), -1)
+    S[np.diag_indices(n)] = rng.uniform(0.5, 2.0, n)
+    S = S @ S.T
+    b = rng.standard_normal(n)
+    rows = np.concatenate([rng.choice(n - 64, 256, replace=False), np.arange(n - 64, n)])
+    with P.Context(cnp, n_cams, 4, 8) as c:
+        out = []
+        for _ in range(2):
+            c.load_S(S, b)
+            ok, x = c.factor_only()
+            assert ok
+            out.append(x.copy())
+        assert np.array_equal(*out)
+        check_factor_and_solution(S, b, out[0], np.tril(c.buffer("L").reshape(n, n)), rows)
+
+
 # together more workgroups than compute units (256): 2 x 136, 4 x 66
 @pytest.mark.parametrize("cnp,n_cams,contexts", [(16, 64, 2), (16, 44, 4)])
 def test_dense_solves_side_by_side(P, gpu, cnp, n_cams, contexts):
