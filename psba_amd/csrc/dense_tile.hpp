@@ -1,6 +1,6 @@
 // 64 x 64 FP64 tiles of the dense factorisation: the factor of a diagonal tile
 // with its inverse, and the fragment layouts in which tiles meet the matrix
-// instructions.  Used by the single-problem and the batched solver.
+// instructions.  Used by k_chol.hip.
 //
 // Fragments.  v_mfma_f64_16x16x4 takes A[row = l % 16][k = l / 16] and
 // B[k = l / 16][col = l % 16] from lane l and leaves C[4 r + l / 16][l % 16] in
@@ -105,7 +105,7 @@ struct ElimStep {
   }
 };
 
-// What tile_factor works on (LDS).  Y: in, the tile (lower part); out, the
+// What the factor of a tile (factor_pivots, factor_blocks, factor_last) works on (LDS).  Y: in, the tile (lower part); out, the
 // factor L~ with its columns not yet scaled (L = L~ / sqrt(d)) below the 16 x 16
 // diagonal blocks, which keep what they held before their own elimination
 // (L's own diagonal blocks: factor_block).  W: out, the rows of L~^-T (row i
@@ -122,8 +122,7 @@ struct FactorLds {
 // prog's words: wave 0's pivots (base + 4 b + g + 1 after four columns g of block
 // b), waves 1, 2, 3 and 7's blocks (base + b + 1), waves 5 and 6's last block
 // column (base + 1), and word 8: base + 1 if a pivot of this tile was not positive.
-enum { kProgPivot = 0, kProgBad = 8, kProgWords = 9 };
-constexpr int kFactorWaves = 8;
+enum { kProgPivot = 0, kProgBad = 8 };
 
 // Progress within the workgroup goes through LDS words rather than barriers, so
 // that no wave waits for one that does not feed it.  A wave's LDS accesses are
@@ -270,7 +269,7 @@ __device__ __forceinline__ void factor_last(const FactorLds& m, int nkb, int bas
 // block (mb, kb <= mb) of a lower triangular tile's fragments
 __device__ __forceinline__ int inv_block(int mb, int kb) { return mb * (mb + 1) / 2 + kb; }
 
-// Block (mb, kb) of M = L^-1 from tile_factor's W and r, by one wave: as operand
+// Block (mb, kb) of M = L^-1 from the factor's W and r, by one wave: as operand
 // fragments (M[16 mb + l % 16][16 kb + 4 (l / 16) + s], values s, s + 1 of lane l as a pair
 // at block * 128 + (s / 2) * 64 + l) in LDS and in global memory, and row-major
 // (64 x 64, nothing above the diagonal blocks) in global memory.
@@ -312,7 +311,7 @@ __device__ __forceinline__ void factor_block_steps(double (&a)[16], double (&r)[
 }
 
 // L's diagonal block b, by one wave: the elimination again, from what Y still
-// holds there (wave 0 of tile_factor has no time to write its rows)
+// holds there (wave 0 has no time to write its rows during the factorisation)
 __device__ __forceinline__ void factor_block(const lds_dbl* Y, int b, double* L, int ld) {
   const int lane = threadIdx.x & 63, li = lane & 15;
   const lds_dvec2* const ar = (const lds_dvec2*)(Y + (16 * b + li) * TS + 16 * b);

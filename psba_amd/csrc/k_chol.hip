@@ -78,27 +78,25 @@ __device__ __forceinline__ void poll(ull* f, ull v, int* fail) {
   }
 }
 
-// The workgroup waits for up to four flags (null: none), one thread each, and may
-// then read what was published before them.
-__device__ __forceinline__ void wait_flags(ull v, int* fail, ull* f0, ull* f1 = nullptr, ull* f2 = nullptr,
-                                           ull* f3 = nullptr) {
+// The workgroup waits for one or two flags, a thread each, and may then read
+// what was published before them.
+__device__ __forceinline__ void wait_flags(ull v, int* fail, ull* f0, ull* f1 = nullptr) {
   const int t = threadIdx.x;
   if (t < 64) {
-    ull* f = t == 0 ? f0 : t == 1 ? f1 : t == 2 ? f2 : t == 3 ? f3 : nullptr;
+    ull* f = t == 0 ? f0 : t == 1 ? f1 : nullptr;
     if (f) poll(f, v, fail);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
 }
 
-// After the workgroup's stores: make them visible and set the flags (null: none).
-__device__ __forceinline__ void publish(ull* f0, ull v, ull* f1 = nullptr) {
+// After the workgroup's stores: make them visible and set the flag.
+__device__ __forceinline__ void publish(ull* f, ull v) {
   drain_stores();
   __syncthreads();  // every wave's stores are in L2
   if (threadIdx.x == 0) {
     release_stores();
-    if (f0) __hip_atomic_store(f0, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (f1) __hip_atomic_store(f1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -473,35 +471,34 @@ __global__ __launch_bounds__(512) void k_chol_solve(double* __restrict__ S, int 
   const bool many = ntiles > G - 2;  // more tiles than workgroups
   // eight waves: row i's share of b (rows i0, i0 + step, .. below i1; row i
   // lies at place i / step) -= L_ik y, with the next two tiles'
-  // loads in flight
+  // loads in flight.  At most 64 rows, a lane each for their flags: all 21 with a
+  // workgroup per tile (T <= 22), kNear or an eighth of 128 with several tiles each.
   auto forward = [&](lds_dbl* b, lds_dbl* y, int k, int i0, int step, int i1) {
-    for (int j0 = i0; j0 < i1; j0 += 64 * step) {
-      const int j1 = min(j0 + 64 * step, i1);
-      if (w == 0) {
-        if (j0 + lane * step < j1) poll(sy.l(j0 + lane * step, k), done, fail);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      }
+    if (i0 >= i1) return;
+    if (w == 0) {
+      if (i0 + lane * step < i1) poll(sy.l(i0 + lane * step, k), done, fail);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    TileRegs<8> t[2][2];
+    auto load = [&](int s, int i) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (i + u * step < i1) t[s][u].load(tile(Lf, i + u * step, k), ld);
+    };
+    auto take = [&](int s, int i) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (i + u * step < i1) t[s][u].rows(y, (lds_dbl*)sm.part[s][u]);
       __syncthreads();
-      TileRegs<8> t[2][2];
-      auto load = [&](int s, int i) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          if (i + u * step < j1) t[s][u].load(tile(Lf, i + u * step, k), ld);
-      };
-      auto take = [&](int s, int i) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          if (i + u * step < j1) t[s][u].rows(y, (lds_dbl*)sm.part[s][u]);
-        __syncthreads();
-        if (w < 2 && i + w * step < j1) b[(i + w * step) / step * NB + lane] -= sm.part[s][w][lane];
-      };
-      load(0, j0);
-      for (int i = j0; i < j1; i += 4 * step) {
-        load(1, i + 2 * step);
-        take(0, i);
-        load(0, i + 4 * step);
-        take(1, i + 2 * step);
-      }
+      if (w < 2 && i + w * step < i1) b[(i + w * step) / step * NB + lane] -= sm.part[s][w][lane];
+    };
+    load(0, i0);
+    for (int i = i0; i < i1; i += 4 * step) {
+      load(1, i + 2 * step);
+      take(0, i);
+      load(0, i + 4 * step);
+      take(1, i + 2 * step);
     }
   };
 

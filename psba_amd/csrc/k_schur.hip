@@ -401,11 +401,11 @@ struct SchurPass {
     for (int k = 0; k < 3; ++k) b[k] = wb[k];
     v = *vi;
   }
-  template <int R, int K>
+  template <int R>
   __device__ __forceinline__ static void outer(double (&acc)[CNP], double y, double bk) {
     if constexpr (R < CNP) {
       fmac_bcast<R>(acc[R], y, bk);
-      outer<R + 1, K>(acc, y, bk);
+      outer<R + 1>(acc, y, bk);
     }
   }
   __device__ __forceinline__ void multiply(double (&acc)[CNP]) {
@@ -420,9 +420,9 @@ struct SchurPass {
     fmac_bcast<2>(y0, v, a[2]);
     fmac_bcast<4>(y1, v, a[2]);
     fmac_bcast<5>(y2, v, a[2]);
-    outer<0, 0>(acc, y0, b[0]);
-    outer<0, 1>(acc, y1, b[1]);
-    outer<0, 2>(acc, y2, b[2]);
+    outer<0>(acc, y0, b[0]);
+    outer<0>(acc, y1, b[1]);
+    outer<0>(acc, y2, b[2]);
   }
 };
 
@@ -430,7 +430,7 @@ template <int CNP>
 __device__ __forceinline__ void schur_group(const int4 grp, const int4* __restrict__ rec,
                                             const double* __restrict__ W, const double* __restrict__ Vinv,
                                             double* __restrict__ part) {
-  constexpr int REC = 3 * CNP, B = 1;  // passes loaded together
+  constexpr int REC = 3 * CNP;
   const int lane = threadIdx.x & 63, row = lane >> 4, l = lane & 15;
   const int n = grp.y - grp.x, np = (n + 3) >> 2;
   // sixteen passes' items, one a lane (lane 16 row + l: pass l's item of the row);
@@ -446,38 +446,33 @@ __device__ __forceinline__ void schur_group(const int4 grp, const int4* __restri
   auto of_pass = [&](const double* x, int p) {
     return (glb_dbl*)__shfl((unsigned long long)x, (lane & 48) + (p & 15), 64);
   };
-  auto load = [&](SchurPass<CNP> (&ps)[B], int p) {
-#pragma unroll
-    for (int u = 0; u < B; ++u)
-      ps[u].load(of_pass(at.wa, p + u) + off, of_pass(at.wb, p + u) + off, of_pass(at.vi, p + u) + voff);
+  auto load = [&](SchurPass<CNP>& ps, int p) {
+    ps.load(of_pass(at.wa, p) + off, of_pass(at.wb, p) + off, of_pass(at.vi, p) + voff);
     __asm__ volatile("" ::: "memory");  // the loads go out ahead of what follows
   };
   double acc[CNP];
 #pragma unroll
   for (int r = 0; r < CNP; ++r) acc[r] = 0.0;
-  auto multiply = [&](SchurPass<CNP> (&ps)[B], int p) {
+  auto multiply = [&](SchurPass<CNP>& ps, int p) {
+    if (4 * (p + 1) > n) {
+      const bool on = 4 * p + row < n;
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (4 * (p + u + 1) > n) {
-        const bool on = 4 * (p + u) + row < n;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) ps[u].b[k] = on ? ps[u].b[k] : 0.0;
-      }
-      ps[u].multiply(acc);
+      for (int k = 0; k < 3; ++k) ps.b[k] = on ? ps.b[k] : 0.0;
     }
+    ps.multiply(acc);
   };
-  SchurPass<CNP> x[B], y[B];
+  SchurPass<CNP> x, y;
   load(x, 0);
 #pragma unroll 1
-  for (int p = 0; p < np; p += 2 * B) {
-    load(y, p + B);
+  for (int p = 0; p < np; p += 2) {
+    load(y, p + 1);
     multiply(x, p);
-    if (((p + 2 * B) & 15) == 0) {
+    if (((p + 2) & 15) == 0) {
       at = at_of(ahead);
-      ahead = item(p + 2 * B + 16);
+      ahead = item(p + 18);
     }
-    load(x, p + 2 * B);
-    if (p + B < np) multiply(y, p + B);
+    load(x, p + 2);
+    if (p + 1 < np) multiply(y, p + 1);
   }
   double* const out = part + (size_t)grp.z * (CNP * CNP);
 #pragma unroll
