@@ -404,8 +404,8 @@ def stage_rates(P, ctx, solve_on, sc, info, r, solve_s):
     ms, n = timed["schur"]
     avg = ms * 1e-3 / max(n, 1)
     flops = 6.0 * C * C * info["n_pair_items"]
-    traffic, src = profiled_traffic("k_schur_ea_groups")
-    out["schur"] = {"kernel": "k_schur_ea_groups", "launches": n, "avg_launch_us": avg * 1e6, "flops_per_launch": flops,
+    traffic, src = profiled_traffic("k_schur_ea_rows")
+    out["schur"] = {"kernel": "k_schur_ea_rows", "launches": n, "avg_launch_us": avg * 1e6, "flops_per_launch": flops,
                     "achieved_TFLOPs": flops / avg / 1e12, "frac_of_fp64_peak": flops / avg / 1e12 / FP64_PEAK_TFLOPS,
                     "traffic": traffic, "traffic_source": src}
     ms, n = timed["backsub"]

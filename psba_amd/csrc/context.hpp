@@ -91,11 +91,9 @@ struct psba_ctx {
   int n_lblocks = 0;            // nc*(nc+1)/2 lower block positions
   int* lblock_pair = nullptr;   // pair index of each lower block position or -1
   int* schunk_order = nullptr;  // launch order of the pair chunks (schunk_launch_key)
-  // schur_rows: the items as (obs in camera k, obs in camera l, point, 0), and groups of
-  // up to schur_group consecutive chunks of a pair in launch order: (first item,
-  // end, first chunk, 0) (built by build_schur_slots)
-  int4 *item_rec = nullptr, *sgroup = nullptr;
-  int schur_group = 1, n_sgroup = 0;
+  // schur_rows: the items as (obs in camera k, obs in camera l, point, 0), and the
+  // chunks in launch order as (first item, end, chunk, 0) (built by build_schur_slots)
+  int4 *item_rec = nullptr, *schunk_rec = nullptr;
   // otherwise: the pair chunks' items in launch order, kPairChunk records per launch
   // slot: (obs in camera k, obs in camera l, point, chunk), then (-1, -1, -1,
   // chunk) past the chunk's items; what k_schur_chunks reads first, at an
@@ -111,7 +109,7 @@ struct psba_ctx {
   double entry_cost = 0;        // SSE at the entry of the last psba_levmar call
 
   bool mixed() const { return precision == PSBA_PREC_MIXED; }
-  // the Schur products go by groups of 16-lane rows (k_schur_ea_groups), not by chunks
+  // a Schur chunk goes to a wave's 16-lane rows (k_schur_ea_rows), not through LDS
   bool schur_rows() const { return !mixed() && cnp > 6; }
 
   // work buffers (plain path: FP64; the mixed path uses the *32 FP32 copies of
@@ -197,7 +195,7 @@ int launch_axpby(psba_ctx* c, double* out, double alpha, const double* a, double
 // ---- launchers (k_schur.hip) ----
 int launch_schur(psba_ctx* c, double mu);                 // S (lower), ea
 int build_point_order(psba_ctx* c);                        // pt_order (index builds)
-int build_schur_slots(psba_ctx* c);                        // item_rec and sgroup or slot_items, cchunk_rec (index builds)
+int build_schur_slots(psba_ctx* c);                        // item_rec and schunk_rec or slot_items, cchunk_rec (index builds)
 int launch_ea_rhs(psba_ctx* c, const double* ga, const double* z, double* out);  // ga - sum W z
 
 // ---- launchers (k_chol.hip) ----

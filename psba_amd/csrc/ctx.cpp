@@ -69,7 +69,7 @@ static void free_index(psba_ctx* c) {
   dfree(c->schunk_order);
   dfree(c->slot_items);
   dfree(c->item_rec);
-  dfree(c->sgroup);
+  dfree(c->schunk_rec);
   dfree(c->cchunk_rec);
   dfree(c->pt_order);
   dfree(c->lblock_pair);
@@ -468,7 +468,7 @@ int alloc_index(psba_ctx* c, long nitems, int npairs, int n_cchunk, int n_schunk
   PSBA_TRY(dalloc(&c->schunk_order, n_schunk));
   if (c->schur_rows()) {
     PSBA_TRY(dalloc(&c->item_rec, (size_t)nitems));
-    PSBA_TRY(dalloc(&c->sgroup, (size_t)n_schunk));
+    PSBA_TRY(dalloc(&c->schunk_rec, (size_t)n_schunk));
   } else {
     PSBA_TRY(dalloc(&c->slot_items, (size_t)n_schunk * kPairChunk));
   }

@@ -411,33 +411,13 @@ __global__ void k_item_recs(const int2* __restrict__ items, const int* __restric
   rec[i] = make_int4(o.x, o.y, obs_pt[o.x], 0);
 }
 
-// the pair of chunk b: psp[q] <= b < psp[q + 1]
-__device__ inline int pair_of_chunk(const int* __restrict__ psp, int npairs, int b) {
-  int lo = 0, hi = npairs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (psp[mid] <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
-// launch slot s starts a group: its chunk is number 0, cpg, 2 cpg, .. of its pair
-__global__ void k_group_flags(const int* __restrict__ order, const int* __restrict__ psp, int npairs, int cpg, int n,
-                              int* __restrict__ flag) {
+// the chunk of each launch slot: its items and its number
+__global__ void k_schunk_recs(const int* __restrict__ order, const int* __restrict__ sb, const int* __restrict__ se,
+                              int n, int4* __restrict__ rec) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const int b = order[s];
-  flag[s] = (b - psp[pair_of_chunk(psp, npairs, b)]) % cpg == 0;
-}
-
-__global__ void k_groups(const int* __restrict__ order, const int* __restrict__ psp, int npairs, int cpg, int n,
-                         const int* __restrict__ sb, const int* __restrict__ se, const int* __restrict__ flag,
-                         const int* __restrict__ pos, int4* __restrict__ grp) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n || !flag[s]) return;
-  const int b = order[s], q = pair_of_chunk(psp, npairs, b);
-  grp[pos[s]] = make_int4(sb[b], se[min(b + cpg, psp[q + 1]) - 1], b, 0);
+  rec[s] = make_int4(sb[b], se[b], b, 0);
 }
 
 __global__ void k_cchunk_recs(const int* __restrict__ cam_obs, const int* __restrict__ cb, const int* __restrict__ ce,
@@ -454,10 +434,6 @@ __global__ void k_cchunk_recs(const int* __restrict__ cam_obs, const int* __rest
   }
 }
 
-// Chunks per group of the FP64 Schur products: a group's wave sums as many items
-// as leave the device full several times over (it holds about 5000 such waves).
-static int schur_group_chunks(int n_schunk) { return n_schunk >= 20000 ? 4 : n_schunk >= 10000 ? 2 : 1; }
-
 // The Schur items' records in launch order and the camera chunks'
 // records, from the finished index (host or device build alike).
 int build_schur_slots(psba_ctx* c) {
@@ -467,32 +443,14 @@ int build_schur_slots(psba_ctx* c) {
     hipLaunchKernelGGL(k_cchunk_recs, dim3((unsigned)(((long)c->n_cchunk * ch + 255) / 256)), dim3(256), 0, st,
                        c->cam_obs, c->cchunk_begin, c->cchunk_end, c->obs_pt, c->n_cchunk, ch, c->cchunk_rec);
   const int n = c->n_schunk;
-  c->n_sgroup = 0;
-  if (n > 0 && !c->schur_rows())
-    hipLaunchKernelGGL(k_slot_items, dim3((unsigned)(((long)n * kPairChunk + 255) / 256)), dim3(256), 0, st,
-                       c->schunk_order, c->schunk_begin, c->schunk_end, c->pair_items, c->obs_pt, n, c->slot_items);
   if (n > 0 && c->schur_rows()) {
-    c->schur_group = schur_group_chunks(n);
-    DevBuf<int> flag, pos;
-    Scratch tmp;
-    size_t tb = 0;
-    PSBA_TRY(flag.alloc(n));
-    PSBA_TRY(pos.alloc(n));
-    const dim3 g((unsigned)((n + 255) / 256));
     hipLaunchKernelGGL(k_item_recs, dim3((unsigned)((c->n_items + 255) / 256)), dim3(256), 0, st, c->pair_items,
                        c->obs_pt, c->n_items, c->item_rec);
-    hipLaunchKernelGGL(k_group_flags, g, dim3(256), 0, st, c->schunk_order, c->pair_schunk_ptr, c->npairs,
-                       c->schur_group, n, flag.p);
-    PSBA_HIP_TRY(rocprim::exclusive_scan(nullptr, tb, flag.p, pos.p, 0, (size_t)n, rocprim::plus<int>(), st));
-    PSBA_TRY(tmp.ensure(tb));
-    PSBA_HIP_TRY(rocprim::exclusive_scan(tmp.p, tb, flag.p, pos.p, 0, (size_t)n, rocprim::plus<int>(), st));
-    hipLaunchKernelGGL(k_groups, g, dim3(256), 0, st, c->schunk_order, c->pair_schunk_ptr, c->npairs, c->schur_group,
-                       n, c->schunk_begin, c->schunk_end, flag.p, pos.p, c->sgroup);
-    int last[2];
-    PSBA_HIP_TRY(hipMemcpyAsync(&last[0], pos.p + n - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    PSBA_HIP_TRY(hipMemcpyAsync(&last[1], flag.p + n - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    PSBA_HIP_TRY(hipStreamSynchronize(st));
-    c->n_sgroup = last[0] + last[1];
+    hipLaunchKernelGGL(k_schunk_recs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, c->schunk_order,
+                       c->schunk_begin, c->schunk_end, n, c->schunk_rec);
+  } else if (n > 0) {
+    hipLaunchKernelGGL(k_slot_items, dim3((unsigned)(((long)n * kPairChunk + 255) / 256)), dim3(256), 0, st,
+                       c->schunk_order, c->schunk_begin, c->schunk_end, c->pair_items, c->obs_pt, n, c->slot_items);
   }
   PSBA_HIP_TRY(hipGetLastError());
   PSBA_HIP_TRY(hipStreamSynchronize(st));

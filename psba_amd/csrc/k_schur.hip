@@ -215,8 +215,7 @@ __global__ __launch_bounds__(256) void k_schur_chunks(const int2* __restrict__ i
 }
 
 // one block per lower block position (k >= l) of S, including empty ones
-// Blocks [0, nlb) write the lower block positions (a pair's partials lie at its
-// chunks 0, cpg, 2 cpg, ..); the remaining blocks
+// Blocks [0, nlb) write the lower block positions; the remaining blocks
 // rewrite the padding rows n..n_pad-1 as identity rows (a failed
 // factorisation may have left anything there).
 template <int CNP, typename R>
@@ -224,7 +223,7 @@ __device__ __forceinline__ void schur_finish_block(int b, const int* __restrict_
                                                    const int* __restrict__ psp, const R* __restrict__ part,
                                                    const double* __restrict__ U, const unsigned char* __restrict__ fix,
                                                    double mu, const double* __restrict__ mu_p, int ld, int nlb, int n,
-                                                   int cpg, double* __restrict__ S) {
+                                                   double* __restrict__ S) {
   constexpr int C2 = CNP * CNP;
   if (mu_p) mu = *mu_p;
   if (b >= nlb) {
@@ -240,11 +239,7 @@ __device__ __forceinline__ void schur_finish_block(int b, const int* __restrict_
   for (int t = threadIdx.x; t < C2; t += blockDim.x) {
     const int r = t / CNP, cc = t - r * CNP;
     double acc = 0.0;
-    if (q >= 0) {
-      const int h0 = psp[q];
-      acc = ordered_sum_few(0, (psp[q + 1] - h0 + cpg - 1) / cpg,
-                            [&](int h) { return (double)part[(size_t)(h0 + h * cpg) * C2 + t]; });
-    }
+    if (q >= 0) acc = ordered_sum_few(psp[q], psp[q + 1], [&](int h) { return (double)part[(size_t)h * C2 + t]; });
     double val;
     if (k == l) {
       double u = U[(size_t)k * C2 + t];
@@ -373,12 +368,11 @@ __global__ __launch_bounds__(256) void k_schur_ea_chunks(const R* __restrict__ W
   }
 }
 
-// The FP64 Schur products of one problem, without LDS: a wave takes a group (up to
-// c->schur_group consecutive chunks of one camera pair) four items at a time, one
-// in each 16-lane row.  Lane l < CNP of a row has row l of W_a and of W_b (and
-// element l < 6 of V^-1); it forms row l of Y = W_a V^-1 and column l of Y W_b^T,
-// with what other lanes hold broadcast inside the multiply-adds (fmac_bcast).
-// The four rows' sums meet at the end of the group.
+// The FP64 Schur products of one problem, without LDS: a wave takes a chunk
+// four items at a time, one in each 16-lane row.  Lane l < CNP of a row has row l
+// of W_a and of W_b (and element l < 6 of V^-1); it forms row l of Y = W_a V^-1
+// and column l of Y W_b^T, with what other lanes hold broadcast inside the
+// multiply-adds (fmac_bcast).  The four rows' sums meet at the end of the chunk.
 //
 // Bound by the rows' lines on their way from L2 to the L1s (an item's two rows
 // and V^-1: 7 lines of 128 B at 9 parameters, 14 TB/s): so nothing else may take
@@ -386,9 +380,16 @@ __global__ __launch_bounds__(256) void k_schur_ea_chunks(const R* __restrict__ W
 // 64 items in LDS for 3 x 3 register blocks (schur_chunk, which mixed precision
 // keeps for its order of sums, and 6 parameters, where a row has only six lanes'
 // work) took LDS bandwidth and four barriers a chunk, and as long to sum its
-// group partials as to form them: 88 cameras with 9 parameters 246 -> 214 us
-// a launch with the e_a chunks, 300 with 9 314 -> 230, 54 with 11 18.5 -> 13.8, 30
-// with 16 18.6 -> 13.9; with 6 parameters it would be 51 -> 70 (138 cameras).
+// group partials as to form them.  Staged -> so, a launch with the e_a chunks, us,
+// with 9 parameters: 40 cameras x 4,000 points 22.8 -> 19.5, 40 x 32,000 89.7 -> 84.6, 88
+// x 24,000 94.4 -> 85.3, 88 x 64,298 225.8 -> 196.3, 300 x 10,000 115 -> 80, 300 x 40,000
+// 290 -> 234; with 11, 30 x 30,000 61 -> 44; with 16, 96 -> 49.  Below some 1,000 chunks
+// a wave's chain shows, and it takes up to 1 us longer (10 x 300: 8.7 -> 9.8).
+// With 6 parameters it would be 51 -> 70 (138 cameras).  Two and four chunks of a
+// pair to a wave (fewer sums at the end, but fewer waves, and the launch order's
+// point ranges left behind) took 92.8 and 110.6 us where one took 89.7 (40 x
+// 32,000), 95.3 and 115.7 for 91.8 (88 x 24,000), 242 and 228 for 225 (88 x 64,298), and
+// gained only with two at 300 x 40,000 (256 for 270).
 typedef const __attribute__((address_space(1))) double glb_dbl;  // (a pointer that went through a shuffle)
 
 template <int CNP>
@@ -427,27 +428,24 @@ struct SchurPass {
 };
 
 template <int CNP>
-__device__ __forceinline__ void schur_group(const int4 grp, const int4* __restrict__ rec,
-                                            const double* __restrict__ W, const double* __restrict__ Vinv,
-                                            double* __restrict__ part) {
+__device__ __forceinline__ void schur_rows(const int4 chunk, const int4* __restrict__ rec,
+                                           const double* __restrict__ W, const double* __restrict__ Vinv,
+                                           double* __restrict__ part) {
+  static_assert(kPairChunk <= 64, "a lane an item");
   constexpr int REC = 3 * CNP;
   const int lane = threadIdx.x & 63, row = lane >> 4, l = lane & 15;
-  const int n = grp.y - grp.x, np = (n + 3) >> 2;
-  // sixteen passes' items, one a lane (lane 16 row + l: pass l's item of the row);
-  // past the end the last one, not counted
-  const int4* const r0 = rec + grp.x;
-  auto item = [&](int p0) { return r0[min(4 * (p0 + l) + row, n - 1)]; };
-  struct At { const double *wa, *wb, *vi; };
-  auto at_of = [&](const int4& r) { return At{W + (size_t)r.x * REC, W + (size_t)r.y * REC, Vinv + (size_t)r.z * 6}; };
-  int4 ahead = item(0);
-  At at = at_of(ahead);
-  ahead = item(16);
+  const int n = chunk.y - chunk.x, np = (n + 3) >> 2;
+  // the passes' items, one a lane (lane 16 row + l: pass l's item of the row); past
+  // the end the last one, not counted
+  const int4 item = rec[chunk.x + min(4 * l + row, n - 1)];
+  const double *const wa = W + (size_t)item.x * REC, *const wb = W + (size_t)item.y * REC,
+               *const vi = Vinv + (size_t)item.z * 6;
   const int off = 3 * min(l, CNP - 1), voff = min(l, 5);
   auto of_pass = [&](const double* x, int p) {
     return (glb_dbl*)__shfl((unsigned long long)x, (lane & 48) + (p & 15), 64);
   };
   auto load = [&](SchurPass<CNP>& ps, int p) {
-    ps.load(of_pass(at.wa, p) + off, of_pass(at.wb, p) + off, of_pass(at.vi, p) + voff);
+    ps.load(of_pass(wa, p) + off, of_pass(wb, p) + off, of_pass(vi, p) + voff);
     __asm__ volatile("" ::: "memory");  // the loads go out ahead of what follows
   };
   double acc[CNP];
@@ -467,14 +465,10 @@ __device__ __forceinline__ void schur_group(const int4 grp, const int4* __restri
   for (int p = 0; p < np; p += 2) {
     load(y, p + 1);
     multiply(x, p);
-    if (((p + 2) & 15) == 0) {
-      at = at_of(ahead);
-      ahead = item(p + 18);
-    }
     load(x, p + 2);
     if (p + 1 < np) multiply(y, p + 1);
   }
-  double* const out = part + (size_t)grp.z * (CNP * CNP);
+  double* const out = part + (size_t)chunk.z * (CNP * CNP);
 #pragma unroll
   for (int r = 0; r < CNP; ++r) {
     double t = acc[r];
@@ -484,27 +478,26 @@ __device__ __forceinline__ void schur_group(const int4 grp, const int4* __restri
   }
 }
 
-// One problem's Schur groups and e_a chunks in one launch, as k_schur_ea_chunks
-// has them; a Schur workgroup's four waves take four neighbouring groups
+// One problem's Schur and e_a chunks in one launch, as k_schur_ea_chunks has
+// them; a Schur workgroup's four waves take four neighbouring chunks of the order
 template <int CNP>
-__global__ __launch_bounds__(256) void k_schur_ea_groups(const double* __restrict__ W,
-                                                         const double* __restrict__ Vinv,
-                                                         double* __restrict__ spart, int ngroup,
-                                                         const int4* __restrict__ grp, const int4* __restrict__ rec,
-                                                         int nb_schur, int neg, int period, int ncc,
-                                                         const int* __restrict__ cb, const int* __restrict__ ce,
-                                                         const double* __restrict__ z, double* __restrict__ epart,
-                                                         const int2* __restrict__ erec) {
+__global__ __launch_bounds__(256) void k_schur_ea_rows(const double* __restrict__ W, const double* __restrict__ Vinv,
+                                                       double* __restrict__ spart, int nchunk,
+                                                       const int4* __restrict__ crec, const int4* __restrict__ rec,
+                                                       int nb_schur, int neg, int period, int ncc,
+                                                       const int* __restrict__ cb, const int* __restrict__ ce,
+                                                       const double* __restrict__ z, double* __restrict__ epart,
+                                                       const int2* __restrict__ erec) {
   constexpr int CH = ea_chunk_obs<CNP>();
   __shared__ double sP[CH * CNP];
   __shared__ int sO[CH], sI[CH];
   const LaunchSlot ls(blockIdx.x, neg, period);
   if (ls.schur >= 0) {
     if (ls.schur >= nb_schur) return;
-    const int wg = xcd_item(ls.schur, (ngroup + 3) >> 2);
-    const int g = 4 * wg + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    if (wg < 0 || g >= ngroup) return;
-    schur_group<CNP>(grp[g], rec, W, Vinv, spart);
+    const int wg = xcd_item(ls.schur, (nchunk + 3) >> 2);
+    const int s = 4 * wg + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (wg < 0 || s >= nchunk) return;
+    schur_rows<CNP>(crec[s], rec, W, Vinv, spart);
   } else if (ls.ea < ncc) {
     ea_chunk<CNP, double>(ls.ea, nullptr, cb, ce, nullptr, W, z, epart, nullptr, nullptr, erec, sP, sO, sI);
   }
@@ -537,12 +530,12 @@ __global__ __launch_bounds__(256) void k_schur_ea_finish(const int* __restrict__
                                                          const int* __restrict__ psp, const R* __restrict__ spart,
                                                          const double* __restrict__ U,
                                                          const unsigned char* __restrict__ fix,
-                                                         const double* __restrict__ mu_p, int ld, int nlb, int n, int cpg,
+                                                         const double* __restrict__ mu_p, int ld, int nlb, int n,
                                                          double* __restrict__ S, int nfin, const int* __restrict__ ccp,
                                                          const R* __restrict__ epart, const double* __restrict__ ga,
                                                          int nc, double* __restrict__ ea, double mu) {
   if ((int)blockIdx.x < nfin)
-    schur_finish_block<CNP, R>(blockIdx.x, lblock_pair, psp, spart, U, fix, mu, mu_p, ld, nlb, n, cpg, S);
+    schur_finish_block<CNP, R>(blockIdx.x, lblock_pair, psp, spart, U, fix, mu, mu_p, ld, nlb, n, S);
   else
     ea_finish_one<CNP, R>(((int)blockIdx.x - nfin) * blockDim.x + threadIdx.x, ccp, epart, ga, nc, ea, nullptr,
                           nullptr);
@@ -553,8 +546,8 @@ static void run_schur_t(psba_ctx* c, double mu, const R* W, R* schpart, R* eapar
   // the Schur work and the e_a chunks in one launch (the e_a chunks after the
   // first Schur workgroups, so they fill the CUs that the Schur launch's tail
   // leaves idle), then both finishes in one launch
-  constexpr bool kGroups = std::is_same<R, double>::value && CNP > 6;
-  const int nwork = kGroups ? (c->n_sgroup + 3) / 4 : c->n_schunk;
+  constexpr bool kRows = std::is_same<R, double>::value && CNP > 6;
+  const int nwork = kRows ? (c->n_schunk + 3) / 4 : c->n_schunk;
   const int nb_schur = nwork > 0 ? (int)xcd_grid(nwork) : 0;
   const int nsg = (nb_schur + 7) / 8, neg = (c->n_cchunk + 7) / 8;
   if (nsg + neg > 0) {
@@ -563,9 +556,9 @@ static void run_schur_t(psba_ctx* c, double mu, const R* W, R* schpart, R* eapar
     const int period = neg > 0 ? std::max(1, nsg / neg) : 1;
     const int ngroups = neg * (period + 1) + std::max(0, nsg - neg * period);
     probe_begin(c, PSBA_PROBE_SCHUR);
-    if constexpr (kGroups)
-      hipLaunchKernelGGL((k_schur_ea_groups<CNP>), dim3(8 * ngroups), dim3(256), 0, c->stream, W, c->Vinv, schpart,
-                         c->n_sgroup, (const int4*)c->sgroup, (const int4*)c->item_rec, nb_schur, neg, period,
+    if constexpr (kRows)
+      hipLaunchKernelGGL((k_schur_ea_rows<CNP>), dim3(8 * ngroups), dim3(256), 0, c->stream, W, c->Vinv, schpart,
+                         c->n_schunk, (const int4*)c->schunk_rec, (const int4*)c->item_rec, nb_schur, neg, period,
                          c->n_cchunk, c->cchunk_begin, c->cchunk_end, c->z, eapart, (const int2*)c->cchunk_rec);
     else
       hipLaunchKernelGGL((k_schur_ea_chunks<CNP, R>), dim3(8 * ngroups), dim3(256), 0, c->stream, W, c->Vinv,
@@ -576,8 +569,7 @@ static void run_schur_t(psba_ctx* c, double mu, const R* W, R* schpart, R* eapar
   const int nfin = c->n_lblocks + (c->n_pad - c->n), bs = finish_block(CNP);
   hipLaunchKernelGGL((k_schur_ea_finish<CNP, R>), dim3(nfin + ceil_div((long)c->nc * CNP, bs)), dim3(bs), 0,
                      c->stream, c->lblock_pair, c->pair_schunk_ptr, schpart, c->U, c->fix, mu_of(c), c->n_pad,
-                     c->n_lblocks, c->n, kGroups ? c->schur_group : 1, c->S, nfin, c->cam_cchunk_ptr, eapart, c->g,
-                     c->nc, c->ea, mu);
+                     c->n_lblocks, c->n, c->S, nfin, c->cam_cchunk_ptr, eapart, c->g, c->nc, c->ea, mu);
 }
 
 template <int CNP>
