@@ -24,7 +24,7 @@ namespace psba {
 
 constexpr int kCamChunk = 256;   // observations per camera chunk (U/g_a/e_a)
 constexpr int kPairChunk = 64;   // shared points per camera-pair chunk (S)
-constexpr int kLongTrack = 7;    // observations from which on several lanes share a point (back-substitution)
+constexpr int kLongTrack = 7;    // observations from which on several lanes may share a point (shared_points)
 constexpr int kNB = 64;          // dense tile size of the Cholesky / solves
 constexpr int kMaxSolveN = 8192; // largest reduced system the single-block solve holds in LDS
 
@@ -53,6 +53,22 @@ struct LmDev {
   int ntrace, trace_cap, trials, pad_;
 };
 enum { kGateActive = 0, kGateJac = 1, kGateAccept = 2, kGateCount = 4 };
+
+// How many points the FP64 back substitution spreads over seven lane triples each,
+// given the number of tracks of kLongTrack observations or more, their sum and
+// the longest: all of those points, where that shortens the launch.  It takes the
+// longest track's chain of loads, 0.37 us a step, to a seventh, with up to seven
+// times the waves.  Unspread / spread, us: 300 cameras x 40,000 points (6,851 of
+// them long, longest 300) 113 / 28, 88 x 64,298 (13,226, 88) 49 / 24, 30 x 60,000 with
+// 16 parameters (13,291, 20) 41 / 33, 30 x 30,000 (6,613, 20) 31 / 23.  Many tracks that
+// are all short, or all alike, gain nothing: 20,000 of 7 9.6 / 12.5, 60,000 of 8 22.0 /
+// 26.3, 20,000 of 14 14.7 / 15.4, of 20 18.3 / 21.4, 50 cameras x 20,000 points (5,646, 8)
+// 9.0 / 10.2.  A few that are short do: 2,000 of 7 8.4 / 6.5, 10 x 3,000 (1,030, 10) 9.4 / 8.0.
+constexpr long long kFewLong = 2048;
+inline int shared_points(long long n_long, long long sum_long, long long longest) {
+  const bool uneven = longest >= 16 && 2 * longest * n_long >= 3 * sum_long;
+  return n_long <= kFewLong || uneven ? (int)n_long : 0;
+}
 
 struct Timing {
   double jac = 0, schur = 0, factor = 0, solve = 0, backsub = 0, resid = 0, other = 0;
@@ -104,7 +120,7 @@ struct psba_ctx {
   // workgroup index gives (built by build_schur_slots)
   int2* cchunk_rec = nullptr;
   int* pt_order = nullptr;      // points by descending track length (ties: ascending id)
-  int n_long = 0;               // points with kLongTrack observations or more
+  int n_long = 0;               // the first points of pt_order that several lanes share (shared_points)
   double sum_t2 = 0;            // sum over points of track length squared
   double entry_cost = 0;        // SSE at the entry of the last psba_levmar call
 

@@ -536,11 +536,15 @@ int psba_set_index(psba_ctx* c, const int* iidx, const int* jidx) {
   // camera pairs k >= l and their items in ascending point order
   std::vector<long> cnt((size_t)nc * nc, 0);
   double st2 = 0;
-  int n_long = 0;
+  long long n_long = 0, sum_long = 0, longest = 0;
   for (int i = 0; i < np; ++i) {
     int t = pt_ptr[i + 1] - pt_ptr[i];
     st2 += (double)t * t;
-    n_long += t >= kLongTrack;
+    if (t >= kLongTrack) {
+      ++n_long;
+      sum_long += t;
+      longest = std::max<long long>(longest, t);
+    }
     for (int a = pt_ptr[i]; a < pt_ptr[i + 1]; ++a)
       for (int b = pt_ptr[i]; b <= a; ++b) cnt[(size_t)jidx[a] * nc + jidx[b]]++;
   }
@@ -594,7 +598,7 @@ int psba_set_index(psba_ctx* c, const int* iidx, const int* jidx) {
 
   PSBA_TRY(alloc_index(c, nitems, npairs, (int)cb.size(), (int)sb.size()));
   c->sum_t2 = st2;
-  c->n_long = n_long;
+  c->n_long = shared_points(n_long, sum_long, longest);
   auto up = [&](void* dst, const void* src, size_t bytes) -> int {
     if (bytes == 0) return PSBA_OK;
     PSBA_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));

@@ -87,7 +87,7 @@ __global__ void k_chunk_counts(const int* __restrict__ ptr, int n, int CH, int* 
   if (j < n) cnt[j] = (ptr[j + 1] - ptr[j] + CH - 1) / CH;
 }
 
-// items of each point; sums: of t squared, and the number of long tracks
+// items of each point; sums: of t squared; the long tracks' number, sum and longest
 __global__ void k_item_counts(const int* __restrict__ pt_ptr, int np, long long* __restrict__ cnt,
                               unsigned long long* __restrict__ sums) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -95,7 +95,11 @@ __global__ void k_item_counts(const int* __restrict__ pt_ptr, int np, long long*
   const long long t = pt_ptr[i + 1] - pt_ptr[i];
   cnt[i] = t * (t + 1) / 2;
   if (t) atomicAdd(sums, (unsigned long long)(t * t));
-  if (t >= kLongTrack) atomicAdd(sums + 1, 1ull);
+  if (t >= kLongTrack) {
+    atomicAdd(sums + 1, 1ull);
+    atomicAdd(sums + 2, (unsigned long long)t);
+    atomicMax(sums + 3, (unsigned long long)t);
+  }
 }
 
 // launch key of each pair chunk (its first item's cameras and point)
@@ -263,14 +267,14 @@ int psba_set_index_device(psba_ctx* c, const int* iidx, const int* jidx) {
   DevBuf<unsigned long long> sums;
   PSBA_TRY(icnt.alloc(np));
   PSBA_TRY(ioff.alloc(np));
-  PSBA_TRY(sums.alloc(2));
-  IX_TRY(hipMemsetAsync(sums.p, 0, sizeof(unsigned long long) * 2, st));
+  PSBA_TRY(sums.alloc(4));
+  IX_TRY(hipMemsetAsync(sums.p, 0, sizeof(unsigned long long) * 4, st));
   hipLaunchKernelGGL(k_item_counts, grid(np), dim3(256), 0, st, ptptr.p, np, icnt.p, sums.p);
   IX_TRY(rocprim::exclusive_scan(nullptr, tb, icnt.p, ioff.p, 0LL, (size_t)np, rocprim::plus<long long>(), st));
   PSBA_TRY(tmp.ensure(tb));
   IX_TRY(rocprim::exclusive_scan(tmp.p, tb, icnt.p, ioff.p, 0LL, (size_t)np, rocprim::plus<long long>(), st));
   long long h_last[2] = {0, 0};
-  unsigned long long h_sums[2] = {0, 0};
+  unsigned long long h_sums[4] = {0, 0, 0, 0};
   int h_cc[2] = {0, 0};
   IX_TRY(hipMemcpyAsync(&h_last[0], ioff.p + (np - 1), sizeof(long long), hipMemcpyDeviceToHost, st));
   IX_TRY(hipMemcpyAsync(&h_last[1], icnt.p + (np - 1), sizeof(long long), hipMemcpyDeviceToHost, st));
@@ -335,7 +339,7 @@ int psba_set_index_device(psba_ctx* c, const int* iidx, const int* jidx) {
   // the context's buffers
   PSBA_TRY(alloc_index(c, (long)nitems, npairs, n_cchunk, n_schunk));
   c->sum_t2 = (double)h_sums[0];
-  c->n_long = (int)h_sums[1];
+  c->n_long = shared_points(h_sums[1], h_sums[2], h_sums[3]);
   IX_TRY(hipMemcpyAsync(c->obs_pt, d_i.p, sizeof(int) * no, hipMemcpyDeviceToDevice, st));
   IX_TRY(hipMemcpyAsync(c->obs_cam, d_j.p, sizeof(int) * no, hipMemcpyDeviceToDevice, st));
   IX_TRY(hipMemcpyAsync(c->pt_ptr, ptptr.p, sizeof(int) * (np + 1), hipMemcpyDeviceToDevice, st));

@@ -651,14 +651,14 @@ int launch_vinv(psba_ctx* c, double mu) {
 constexpr int kBacksubPtsPerWave = 21;
 constexpr int kBacksubLdsDpa = 4096;  // camera parameters that go through LDS (32 KB)
 
-// Points of long tracks (kLongTrack observations and more, first in `order`) get
-// seven times the lanes, three points a wave: each triple of lanes sums every
-// seventh observation, and the seven sums are added in order.  Otherwise the
-// longest track's chain of loads bounds the launch (0.37 us a step): 300 cameras
-// with 9 parameters, longest track 300: 112 -> 28 us; 88 cameras: 44 -> 21; 138
-// cameras with 6: 40 -> 13; 30 with 16, longest track 20: 20 -> 11.  The line: an
-// observation for every triple; at 10, 16 and 24 the 88 cameras take 23, 23 and 25 us, the 30
-// cameras 14, 20 and 20, the 300 27, 27 and 26.
+// The first n_long points of `order` (long tracks, shared_points) get seven times
+// the lanes, three points a wave: each triple of lanes sums every seventh
+// observation, and the seven sums are added in order.  Otherwise the longest track's
+// chain of loads bounds the launch: 300 cameras with 9 parameters, longest track
+// 300: 112 -> 28 us; 88 cameras: 44 -> 21; 138 cameras with 6: 40 -> 13; 30 with 16,
+// longest track 20: 20 -> 11.  Long: an observation for every triple; from 10, 16 and
+// 24 on the 88 cameras take 23, 23 and 25 us, the 30 cameras 14, 20 and 20, the 300 27,
+// 27 and 26.
 constexpr int kLongLanes = 7;
 
 // With LDS_DPA the camera step dp[0..n) is first copied into LDS (dynamic

@@ -116,7 +116,9 @@ def test_generate_idxs_device_scene(P, gpu):
 
 # tracks on both sides of seven observations, from which on several lanes share a point
 @pytest.mark.parametrize("config,kw", [(1, dict(n_cams=9, n_pts=30)), (2, dict(n_cams=6, n_pts=200)),
-                                       (2, dict(n_cams=60, n_pts=700))])
+                                       (2, dict(n_cams=60, n_pts=700)),
+                                       # many: uneven ones, and ones of seven and eight, which are not shared
+                                       (1, dict(cnp=16, n_cams=30, n_pts=12000)), (4, dict(size_class=1))])
 def test_steps_of_long_tracks_are_the_same_with_either_index(P, gpu, config, kw):
     sc = P.Scene(config, 12, **kw)
     out = []

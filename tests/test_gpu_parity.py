@@ -107,6 +107,26 @@ def test_backsub_of_long_tracks(P, O, gpu, config, kw):
     assert rel(g.buffer("EB"), o.buffer("EB")) < 1e-11
 
 
+# many long tracks: uneven ones, which are shared by lanes, and ones of seven and
+# eight, which are not
+@pytest.mark.parametrize("config,kw", [(1, dict(cnp=16, n_cams=30, n_pts=12000)), (4, dict(size_class=1))])
+def test_backsub_of_many_long_tracks(P, O, gpu, config, kw):
+    sc = P.Scene(config, 12, **kw)
+    assert np.sum(np.bincount(sc.iidx) >= 7) > 2048
+    g, o = pair(P, O, sc)
+    O.set_threads(16)
+    g.jacobian_normal(1.0, 1.0)
+    o.jacobian_normal(1.0, 1.0)
+    mu = 1e-3 * o.max_uvdiag()
+    g.schur(mu)
+    o.schur(mu)
+    assert g.factor_solve() and o.factor_solve()
+    g.backsub()
+    o.backsub()
+    assert rel(g.buffer("DP"), o.buffer("DP")) < 1e-9
+    assert rel(g.buffer("EB"), o.buffer("EB")) < 1e-11
+
+
 def test_schur_is_deterministic(P, gpu):
     sc = P.Scene(2, 7, n_pts=4000, n_cams=24)
     a = P.Context.from_scene(sc)
