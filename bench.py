@@ -518,7 +518,7 @@ def main():
     for _ in range(a.warmup):
         solve()
     # HIP events around every launch of the dense factor + solve (the kernel
-    # with the largest share of the solve's device time) on the context's stream
+    # with the longest dependent chain) on the context's stream
     ctx.probe(P.PROBE_FACTOR)
     ctx.probe_read()
     res = []
